@@ -140,6 +140,12 @@ __device__ __forceinline__ float q_split_e4m3(const uint16_t* qrow, bool ok, uin
     return __builtin_ldexpf(1.0f, -sh);
 }
 
+// A two-part launch's tiles of up to this many tokens run as one part: joining
+// the parts costs 1-2 us, about what splitting 8 chunks gains (FP8, 24/4 heads,
+// 6 per workgroup, 128 rows without context 15.1 us, in two parts 16.3; 512
+// rows 29.6 and 27.2).
+constexpr uint32_t kTwoPartTokens = 256;
+
 constexpr uint32_t kTilePageWindow = 1024;   // block-table entries staged in LDS per pass
 
 // LDS bytes of one pipeline stage: K and V of a 32-token chunk (lane-major DMA
@@ -155,7 +161,7 @@ constexpr int kTileStages = 4;   // two pairs of chunks (see the main loop)
 // page and its page id, base address and in-page offset are wave-uniform.
 // Waves per SIMD the register budget targets: 3 with one head per wave, 2
 // with two (the accumulators of 2 heads take 128 registers at D=256).
-constexpr int tile_waves_per_simd(int hpw) { return hpw == 1 ? 3 : 2; }
+constexpr int tile_waves_per_simd(int hpw, int nw = 0) { return nw > 12 ? 4 : hpw == 1 ? 3 : 2; }
 
 // GQA groups that grouped launches take: 1-8 heads per kv head, as head
 // pairs (a 1-head group or the last pair of an odd group computes one head
@@ -224,11 +230,11 @@ constexpr uint32_t kDenseTileUnits = 1024;
 // over blocks of different context lengths otherwise leaves most of its grid
 // empty and the active workgroups unevenly spread over the XCDs. Returns
 // false for a workgroup without work.
-template <int NW, int HPW, int RT>
+template <int NW, int HPW, int RT, int TS>
 __device__ __forceinline__ bool tile_workgroup(const TileParams& p, uint32_t qpk, uint32_t& split,
                                                uint32_t& hpart, uint32_t& kv_head, uint32_t& group) {
     hpart = 0u;
-    if constexpr (RT == 1) {
+    if constexpr (RT == 1 && TS == 1) {
         const uint32_t count = p.n_tiles != 0u ? p.n_tiles : (p.a.rows + kTileRows - 1u) / kTileRows;
         if (p.splits > 1u && (uint64_t)count * p.splits <= kDenseTileUnits) {
             kv_head = blockIdx.x % p.a.kv_heads;
@@ -238,8 +244,9 @@ __device__ __forceinline__ bool tile_workgroup(const TileParams& p, uint32_t qpk
     }
     split = blockIdx.x % p.splits;
     uint32_t rest = blockIdx.x / p.splits;
-    if constexpr (RT > 1) {
-        const uint32_t hparts = (qpk + HPW - 1u) / HPW;
+    if constexpr (RT > 1 || TS > 1) {
+        constexpr uint32_t kPartHeads = RT > 1 ? HPW : NW / TS;
+        const uint32_t hparts = (qpk + kPartHeads - 1u) / kPartHeads;
         hpart = rest % hparts;
         rest /= hparts;
     }
@@ -248,13 +255,48 @@ __device__ __forceinline__ bool tile_workgroup(const TileParams& p, uint32_t qpk
     return true;
 }
 
-template <int FMT, int D, int NW, int HPW, int RT, bool kAl16>
-__global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_kernel(const TileParams p) {
+// LDS of one head's (m, l, O) of 16 rows, as part 1 leaves it for part 0.
+template <int NDB>
+constexpr size_t part_bytes() { return (size_t)NDB * 1024 + 512; }
+
+// Two-part tiles: part 1 (waves past WH) leaves (m, l, O) in LDS, part 0 folds
+// them into its own. All live waves call it after a barrier; false for part 1.
+template <int NDB, int WH>
+__device__ __forceinline__ bool join_parts(uint8_t* lds, uint32_t w, uint32_t lane, bool computes, float& m_run,
+                                           float& l_run, f32x4 (&o)[NDB]) {
+    const bool second = w >= (uint32_t)WH;
+    uint8_t* const at = lds + (w % (uint32_t)WH) * (uint32_t)part_bytes<NDB>();
+    f32x4* const os = reinterpret_cast<f32x4*>(at) + lane;
+    float* const ml = reinterpret_cast<float*>(at + NDB * 1024) + lane;
+    if (second && computes) {
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) os[64 * db] = o[db];
+        ml[0] = m_run;
+        ml[64] = l_run;
+    }
+    __syncthreads();
+    if (second) return false;
+    if (computes) {
+        const float m1 = ml[0], l1 = ml[64];
+        const float m = __builtin_fmaxf(m_run, m1);
+        const float mu = m == -INFINITY ? 0.0f : m;
+        const float a0 = __builtin_amdgcn_exp2f(m_run - mu), a1 = __builtin_amdgcn_exp2f(m1 - mu);
+        l_run = l_run * a0 + l1 * a1;
+        m_run = m;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) o[db] = o[db] * a0 + os[64 * db] * a1;
+    }
+    return true;
+}
+
+template <int FMT, int D, int NW, int HPW, int RT, int TS, bool kAl16>
+__global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW, NW)) void paged_tile_kernel(const TileParams p) {
+    static_assert(TS == 1 || (TS == 2 && RT == 1 && HPW == 1), "parts: one head per wave of one tile");
     static_assert(RT == 1 || RT == NW, "grouped tiles: one wave per tile");
     static_assert(FMT == kFmtBf16 || FMT == kFmtFp8, "PSQ tiles: paged_tile_psq_group_kernel");
     constexpr int KVB = FMT == kFmtBf16 ? 2 : 1;   // bytes per value
     constexpr int CB = code_bytes<FMT, D>();       // K (V) bytes of one token's head slice
-    constexpr int WH = NW / RT;          // waves along the heads of one tile
+    constexpr int WH = NW / RT / TS;     // waves along the heads of one tile
     constexpr int H = 2;                 // 16-token halves per chunk
     constexpr int CT = 16 * H;           // tokens per chunk
     constexpr int NL = CB / 64;          // 16 B DMA pieces per lane per half
@@ -291,7 +333,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
     const uint32_t qpk = a.q_heads / a.kv_heads;
 
     uint32_t split, hpart, kv_head, group;
-    if (!tile_workgroup<NW, HPW, RT>(p, qpk, split, hpart, kv_head, group)) return;
+    if (!tile_workgroup<NW, HPW, RT, TS>(p, qpk, split, hpart, kv_head, group)) return;
     const uint32_t rt = RT > 1 ? w : 0u;
     const uint32_t tile = group * RT + rt;
     // the group's first tile names the sequence (workgroup-uniform)
@@ -360,8 +402,13 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
     // Everything above is uniform over the workgroup, so all waves reach the
     // barriers below; a wave past the last query head of the group only
     // issues its share of the DMAs.
-    const uint32_t hbase = RT > 1 ? hpart * HPW : w * HPW;   // first head (group index)
-    const bool computes = hbase < qpk && wave_vis > 0u;
+    // first head (group index)
+    const uint32_t hbase = RT > 1 ? hpart * HPW : TS > 1 ? hpart * (uint32_t)WH + w % (uint32_t)WH : w * HPW;
+    // TS == 2: this wave's part, the chunks of its parity. A short range is one
+    // part: the waves of the other only stage
+    const uint32_t part = TS > 1 ? __builtin_amdgcn_readfirstlane(w / (uint32_t)WH) : 0u;
+    const uint32_t parts = TS > 1 && __builtin_amdgcn_readfirstlane(t_end - t_begin) > kTwoPartTokens ? 2u : 1u;
+    const bool computes = hbase < qpk && wave_vis > 0u && part < parts;
 
     if (tid == 0) bad_lds = 0u;
 
@@ -795,6 +842,19 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
                          __attribute__((always_inline)) {
             issue(c + 2 * CT, next);
             issue(c + 3 * CT, next + STAGE);
+            if constexpr (TS > 1) {
+                if (!computes) return;
+#pragma unroll 1
+                for (uint32_t u = part; u < 2u; u += parts) {
+                    const uint32_t cu = c + u * CT;
+                    if (cu >= te || cu >= wave_vis) break;
+                    if (cu + CT <= wave_vis_min && cu + CT <= te)
+                        consume(cu, cur + u * STAGE, std::true_type{});
+                    else
+                        consume(cu, cur + u * STAGE, std::false_type{});
+                }
+                return;
+            }
             if (computes && c < wave_vis) {
                 if (c + CT <= wave_vis_min && c + CT <= te)
                     consume(c, cur, std::true_type{});
@@ -820,6 +880,9 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
         wait_vmcnt<0>();
     }
     __syncthreads();
+    if constexpr (TS > 1) {
+        if (parts == 2u && !join_parts<NDB, WH>(lds, w, lane, computes, m_run[0], l_run[0], o[0])) return;
+    }
     if (!computes) return;
     float* part_row = nullptr;
     if (p.partials != nullptr)
@@ -894,10 +957,10 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
 template <int FMT>
 constexpr int pg_code_stages() { return FMT == kFmtPsq4 ? 3 : 2; }
 
-template <int FMT, int D>
+template <int FMT, int D, int TS = 1>
 constexpr size_t tile_pg_lds_bytes() {
-    return (size_t)kTilePageWindow * 4 + (size_t)pg_code_stages<FMT>() * tile_stage_bytes<FMT, D>() +
-           (size_t)tile_stage_bytes<kFmtBf16, D>();
+    return (size_t)kTilePageWindow * 4 + (size_t)pg_code_stages<FMT>() * TS * tile_stage_bytes<FMT, D>() +
+           (size_t)TS * tile_stage_bytes<kFmtBf16, D>();
 }
 
 // RT == kTileGroup (grouped prefill): wave w owns tile w of the group and
@@ -905,8 +968,9 @@ constexpr size_t tile_pg_lds_bytes() {
 // implicit tiles, other group sizes): the NW waves own HPW = 1 head each of
 // one tile. The first 4 waves issue the DMAs; the first 4 (8 at head_dim
 // 256 with 8 waves) dequantize.
-template <int FMT, int D, int NW, int HPW, int RT, bool kAl16>
-__global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_psq_group_kernel(const TileParams p) {
+template <int FMT, int D, int NW, int HPW, int RT, int TS, bool kAl16>
+__global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW, NW)) void paged_tile_psq_group_kernel(const TileParams p) {
+    constexpr int WH = NW / RT / TS;                  // waves along the heads of one tile
     constexpr int H = 2;
     constexpr int CT = 32;
     constexpr int CB = code_bytes<FMT, D>();          // code bytes of one token's head slice
@@ -917,20 +981,22 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
     constexpr int HSC = 16 * CB + 128;                // code half stride
     constexpr int KVC = H * HSC;
     constexpr int SC_BYTES = H * 256;
-    constexpr int CSTAGE = tile_stage_bytes<FMT, D>();
+    constexpr int CSTAGE = tile_stage_bytes<FMT, D>();   // one chunk's codes; a code stage holds TS
+    constexpr int BSTAGE = tile_stage_bytes<kFmtBf16, D>();
+    constexpr int SPW = 4 * TS > NW ? 4 * TS / NW : 1;   // DMA streams (dequantized units) per wave
     constexpr int CS = pg_code_stages<FMT>();
     constexpr int HSB = 16 * 2 * D + 128;             // f16 half stride
     constexpr int KVB_BYTES = H * HSB;
-    constexpr int DPW = NL + 1;
+    constexpr int DPW = SPW * (NL + 1);
     constexpr int kWinBytes = (int)kTilePageWindow * 4;
     // waves that dequantize each chunk: 8 at head_dim 256 with 8 or more
     // waves (one 32-value block per lane), else 4 (D / 128 blocks per lane)
-    constexpr int NDQ = NW >= 8 && D == 256 ? 8 : 4;
-    constexpr int QD = D / NDQ;                       // dims one lane dequantizes per token row
+    constexpr int NDQ = NW >= 8 && (D == 256 || TS > 1) ? 8 : 4;
+    constexpr int QD = TS > 1 ? D / 4 : D / NDQ;                       // dims one lane dequantizes per token row
     // exponent headroom of the dequantized chunk: largest code x 2 x 2^kB
     // (PSQ4 10 x 2 x 2^11 = 40960, PSQ8 448 x 2 x 2^6 = 57344) stays below 65504
     constexpr int kB = FMT == kFmtPsq4 ? 11 : 6;
-    static_assert((RT == NW && HPW == 2) || (RT == 1 && HPW == 1), "tile geometry");
+    static_assert((RT == NW && HPW == 2 && TS == 1) || (RT == 1 && HPW == 1 && TS <= 2), "tile geometry");
     static_assert(NW >= 4 && NS % 2 == 0 && D % 128 == 0, "geometry");
 
     extern __shared__ __align__(16) uint8_t lds[];
@@ -944,7 +1010,7 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
     const uint32_t qpk = a.q_heads / a.kv_heads;
 
     uint32_t split, hpart, kv_head, group;
-    if (!tile_workgroup<NW, HPW, RT>(p, qpk, split, hpart, kv_head, group)) return;
+    if (!tile_workgroup<NW, HPW, RT, TS>(p, qpk, split, hpart, kv_head, group)) return;
     // the group's first tile names the sequence (workgroup-uniform)
     uint32_t g0;
     if (p.n_tiles != 0u) {
@@ -1006,8 +1072,13 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
     const uint64_t scale_layer = (uint64_t)a.layer * a.num_pages;
     // everything above is uniform over the workgroup: all waves reach the
     // barriers below
-    const uint32_t hbase = RT > 1 ? hpart * HPW : w * HPW;   // first head (group index)
-    const bool computes = hbase < qpk && wave_vis > 0u;
+    // first head (group index)
+    const uint32_t hbase = RT > 1 ? hpart * HPW : TS > 1 ? hpart * (uint32_t)WH + w % (uint32_t)WH : w * HPW;
+    // TS == 2: this wave's part, the chunks of its parity. A short range is one
+    // part: the waves of the other only stage
+    const uint32_t part = TS > 1 ? __builtin_amdgcn_readfirstlane(w / (uint32_t)WH) : 0u;
+    const uint32_t parts = TS > 1 && __builtin_amdgcn_readfirstlane(t_end - t_begin) > kTwoPartTokens ? 2u : 1u;
+    const bool computes = hbase < qpk && wave_vis > 0u && part < parts;
     bool hv[HPW];
 #pragma unroll
     for (int i = 0; i < HPW; ++i) hv[i] = hbase + (uint32_t)i < qpk;
@@ -1129,14 +1200,15 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
 
     uint32_t* const win = reinterpret_cast<uint32_t*>(lds);
     uint8_t* const cstages = lds + kWinBytes;
-    uint8_t* const bst = cstages + CS * CSTAGE;       // the f16 chunk
+    uint8_t* const bst = cstages + CS * TS * CSTAGE;  // the f16 chunk (TS == 2: both of a pair)
     const uint32_t wu = __builtin_amdgcn_readfirstlane(w);
     // dequantization: wave w < NDQ takes (kind, half, dim part) = ((w / 2) % 2,
     // w % 2, w / 4), lane (t, q) token t, dims [QD j, QD (j + 1)) with j =
     // (NDQ / 4) q + w / 4. The LDS serves 8 lanes of a 16 B access per clock;
     // they are 8 tokens of one 16 B column, whose rows sit 16 B apart, so the
     // 8 accesses hit distinct banks.
-    const uint32_t dq = (uint32_t)(NDQ / 4) * g + (w >> 2);
+    // TS == 2: wave w (and w + 4 with 4 waves) the chunk w / 4 of the pair, QD = D / 4.
+    const uint32_t dq = TS > 1 ? g : (uint32_t)(NDQ / 4) * g + (w >> 2);
     const uint32_t d_kind = (w >> 1) & 1u, d_half = w & 1u, d_tok = n;
 
     for (uint32_t wp = pb; wp < pe; wp += kTilePageWindow) {
@@ -1148,39 +1220,44 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
         const uint32_t te = min(wp_end * P, t_end);
         if (ts >= te) continue;
         const uint32_t t_last = te - 1u;
-        const uint32_t K = (te - ts + CT - 1u) / CT;
+        const uint32_t K = (te - ts + TS * CT - 1u) / (TS * CT);
         const uint32_t tok_bytes = a.kv_heads * (uint32_t)CB;
         // wave wu: stream (K | V, half wu % 2) of chunk ci: NL code pieces and
         // dword g of each token's block scales (lane groups past SW repeat one)
         auto issue = [&](uint32_t ci, uint8_t* st) __attribute__((always_inline)) {
-            if (NW > 4 && wu >= 4u) return;
-            const uint32_t c = ts + ci * CT;
-            const uint32_t hf = wu % (uint32_t)H;
-            const uint32_t kind = wu / (uint32_t)H;
-            const uint32_t tau = min(c + hf * 16u + n, t_last);
-            uint32_t page, off;
-            if constexpr (kAl16) {
-                const uint32_t hb = min(c + hf * 16u, t_last);
-                const uint32_t pi = hb / P;
-                page = __builtin_amdgcn_readfirstlane(win[pi - wp]);
-                off = tau - pi * P;
-            } else {
-                page = win[tau / P - wp];
-                off = tau % P;
-            }
-            const bool inv = page >= a.num_pages;
-            if (inv) bad_lds = 1u;
-            const uint32_t pg = inv ? 0u : page;
-            const uint64_t slice0 = ((scale_layer + pg) * P * a.kv_heads + kv_head) * (uint64_t)CB;
-            const uint8_t* src = (kind == 0u ? p.k_pool : p.v_pool) + slice0;
-            uint8_t* dst = st + kind * KVC + hf * HSC;
-            const uint32_t lo = off * tok_bytes + g * 16u;
+            if (NW > 4 * TS && wu >= 4u * TS) return;
 #pragma unroll
-            for (int i = 0; i < NL; ++i) load_lds<16>(src + (lo + i * 64u), dst + i * 1024);
-            const uint64_t si = ((scale_layer + pg) * P + off) * a.kv_heads + kv_head;
-            const uint8_t* sbase = reinterpret_cast<const uint8_t*>(kind == 0u ? p.k_scale : p.v_scale);
-            load_lds<4>(sbase + si * (2u * D / 32u) + 4u * min(g, (uint32_t)SW - 1u),
-                        st + 2 * KVC + kind * SC_BYTES + hf * 256);
+            for (int u = 0; u < SPW; ++u) {
+                const uint32_t su = wu + (uint32_t)(u * NW);   // stream: chunk su / 4 of the stage
+                const uint32_t c = ts + (TS > 1 ? ci * TS + su / 4u : ci) * CT;
+                const uint32_t hf = su % (uint32_t)H;
+                const uint32_t kind = TS > 1 ? su / (uint32_t)H % 2u : su / (uint32_t)H;
+                uint8_t* const sst = TS > 1 ? st + su / 4u * CSTAGE : st;
+                const uint32_t tau = min(c + hf * 16u + n, t_last);
+                uint32_t page, off;
+                if constexpr (kAl16) {
+                    const uint32_t hb = min(c + hf * 16u, t_last);
+                    const uint32_t pi = hb / P;
+                    page = __builtin_amdgcn_readfirstlane(win[pi - wp]);
+                    off = tau - pi * P;
+                } else {
+                    page = win[tau / P - wp];
+                    off = tau % P;
+                }
+                const bool inv = page >= a.num_pages;
+                if (inv) bad_lds = 1u;
+                const uint32_t pg = inv ? 0u : page;
+                const uint64_t slice0 = ((scale_layer + pg) * P * a.kv_heads + kv_head) * (uint64_t)CB;
+                const uint8_t* src = (kind == 0u ? p.k_pool : p.v_pool) + slice0;
+                uint8_t* dst = sst + kind * KVC + hf * HSC;
+                const uint32_t lo = off * tok_bytes + g * 16u;
+#pragma unroll
+                for (int i = 0; i < NL; ++i) load_lds<16>(src + (lo + i * 64u), dst + i * 1024);
+                const uint64_t si = ((scale_layer + pg) * P + off) * a.kv_heads + kv_head;
+                const uint8_t* sbase = reinterpret_cast<const uint8_t*>(kind == 0u ? p.k_scale : p.v_scale);
+                load_lds<4>(sbase + si * (2u * D / 32u) + 4u * min(g, (uint32_t)SW - 1u),
+                            sst + 2 * KVC + kind * SC_BYTES + hf * 256);
+            }
         };
         // code stage st -> f16 chunk: this lane's token row, QD dims, each
         // value scaled by 2^(kB + 127 - Ek) (K) or 2^(kB + 127 - Ev) (V)
@@ -1368,8 +1445,29 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
         auto step = [&](uint32_t k, uint8_t* __restrict__ next, const uint8_t* __restrict__ cur,
                         uint8_t* __restrict__ bchunk) __attribute__((always_inline)) {
             issue(k + (uint32_t)CS - 1u, next);
-            dequant(cur, bchunk);
+            if constexpr (TS > 1) {
+#pragma unroll
+                for (int u = 0; u < SPW; ++u) {
+                    const uint32_t ch = (wu + (uint32_t)(u * NW)) >> 2;
+                    dequant(cur + ch * CSTAGE, bchunk + ch * BSTAGE);
+                }
+            } else {
+                dequant(cur, bchunk);
+            }
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if constexpr (TS > 1) {
+                if (!computes) return;
+#pragma unroll 1
+                for (uint32_t u = part; u < 2u; u += parts) {
+                    const uint32_t cu = ts + (k * TS + u) * CT;
+                    if (cu >= te || cu >= wave_vis) break;
+                    if (cu + CT <= wave_vis_min && cu + CT <= te)
+                        consume(cu, bchunk + u * BSTAGE, std::true_type{});
+                    else
+                        consume(cu, bchunk + u * BSTAGE, std::false_type{});
+                }
+                return;
+            }
             const uint32_t c = ts + k * CT;
             if (computes && c < wave_vis) {
                 if (c + CT <= wave_vis_min && c + CT <= te)
@@ -1379,17 +1477,20 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
             }
         };
 #pragma unroll
-        for (int l = 0; l < CS - 1; ++l) issue((uint32_t)l, cstages + l * CSTAGE);
+        for (int l = 0; l < CS - 1; ++l) issue((uint32_t)l, cstages + l * TS * CSTAGE);
         for (uint32_t k = 0; k < K; ++k) {
             // chunk k landed (CS - 2 later chunks outstanding); every wave is
             // done with the f16 chunk and with code stage (k - 1) % CS
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((CS - 2) * DPW) : "memory");
-            step(k, cstages + ((k + (uint32_t)CS - 1u) % (uint32_t)CS) * CSTAGE, cstages + (k % (uint32_t)CS) * CSTAGE,
-                 bst);
+            step(k, cstages + ((k + (uint32_t)CS - 1u) % (uint32_t)CS) * (TS * CSTAGE),
+                 cstages + (k % (uint32_t)CS) * (TS * CSTAGE), bst);
         }
         wait_vmcnt<0>();   // the DMAs of chunks nobody reads
     }
     __syncthreads();
+    if constexpr (TS > 1) {
+        if (parts == 2u && !join_parts<NDB, WH>(lds, w, lane, computes, m_run[0], l_run[0], o[0])) return;
+    }
     if (!computes) return;
     float* part_row = nullptr;
     if (p.partials != nullptr)
@@ -1450,22 +1551,29 @@ __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW)) void paged_tile_
     }
 }
 
-template <int FMT, int D, int NW, int HPW, int RT, bool kAl16>
+// LDS of a launch: its pipeline, where two parts of wh heads join afterwards.
+template <int D, int TS>
+constexpr size_t with_join(size_t lds, int wh) {
+    const size_t join = TS > 1 ? (size_t)wh * part_bytes<D / 16>() : 0;
+    return lds > join ? lds : join;
+}
+
+template <int FMT, int D, int NW, int HPW, int RT, int TS, bool kAl16>
 hipError_t launch_tile_pg_t(const TileParams& p, uint64_t grid, hipStream_t stream) {
-    constexpr size_t lds_bytes = tile_pg_lds_bytes<FMT, D>();
+    constexpr size_t lds_bytes = with_join<D, TS>(tile_pg_lds_bytes<FMT, D, TS>(), NW / TS);
     static std::atomic<uint64_t> lds_ready{0};
     const hipError_t attr = allow_full_lds(
-        reinterpret_cast<const void*>(&paged_tile_psq_group_kernel<FMT, D, NW, HPW, RT, kAl16>), lds_ready);
+        reinterpret_cast<const void*>(&paged_tile_psq_group_kernel<FMT, D, NW, HPW, RT, TS, kAl16>), lds_ready);
     if (attr != hipSuccess) return attr;
-    hipLaunchKernelGGL((paged_tile_psq_group_kernel<FMT, D, NW, HPW, RT, kAl16>), dim3((uint32_t)grid),
+    hipLaunchKernelGGL((paged_tile_psq_group_kernel<FMT, D, NW, HPW, RT, TS, kAl16>), dim3((uint32_t)grid),
                        dim3(NW * 64), lds_bytes, stream, p);
     return hipGetLastError();
 }
 
-template <int FMT, int D, int NW, int HPW, int RT>
+template <int FMT, int D, int NW, int HPW, int RT, int TS = 1>
 hipError_t launch_tile_pg(const TileParams& p, uint64_t grid, hipStream_t stream) {
-    return (p.a.page_tokens & 15u) == 0u ? launch_tile_pg_t<FMT, D, NW, HPW, RT, true>(p, grid, stream)
-                                         : launch_tile_pg_t<FMT, D, NW, HPW, RT, false>(p, grid, stream);
+    return (p.a.page_tokens & 15u) == 0u ? launch_tile_pg_t<FMT, D, NW, HPW, RT, TS, true>(p, grid, stream)
+                                         : launch_tile_pg_t<FMT, D, NW, HPW, RT, TS, false>(p, grid, stream);
 }
 
 // kv_dtype: PSK_KV_*. PSQ: head_dim 128 or 256 (every (token, head) code
@@ -1491,25 +1599,60 @@ bool tile_shape_ok(const psk_paged_attention_args& c, uint32_t kv_dtype, const v
     return true;
 }
 
-template <int FMT, int D, int NW, int HPW, int RT, bool kAl16>
+template <int FMT, int D, int NW, int HPW, int RT, int TS, bool kAl16>
 hipError_t launch_tile_t3(const TileParams& p, uint64_t grid, hipStream_t stream) {
-    const size_t lds_bytes = (size_t)kTilePageWindow * 4 + (size_t)kTileStages * tile_stage_bytes<FMT, D>();
+    constexpr size_t lds_bytes = with_join<D, TS>(
+        (size_t)kTilePageWindow * 4 + (size_t)kTileStages * tile_stage_bytes<FMT, D>(), NW / TS);
     if (lds_bytes > 64u * 1024u) {
         // gfx950 has 160 KB of LDS per CU; raise the per-kernel dynamic limit.
         static std::atomic<uint64_t> lds_ready{0};
         const hipError_t attr =
-            allow_full_lds(reinterpret_cast<const void*>(&paged_tile_kernel<FMT, D, NW, HPW, RT, kAl16>), lds_ready);
+            allow_full_lds(reinterpret_cast<const void*>(&paged_tile_kernel<FMT, D, NW, HPW, RT, TS, kAl16>), lds_ready);
         if (attr != hipSuccess) return attr;
     }
-    hipLaunchKernelGGL((paged_tile_kernel<FMT, D, NW, HPW, RT, kAl16>), dim3((uint32_t)grid),
+    hipLaunchKernelGGL((paged_tile_kernel<FMT, D, NW, HPW, RT, TS, kAl16>), dim3((uint32_t)grid),
                        dim3(NW * 64), lds_bytes, stream, p);
     return hipGetLastError();
 }
 
-template <int FMT, int D, int NW, int HPW, int RT = 1>
+template <int FMT, int D, int NW, int HPW, int RT = 1, int TS = 1>
 hipError_t launch_tile_t2(const TileParams& p, uint64_t grid, hipStream_t stream) {
-    return (p.a.page_tokens & 15u) == 0u ? launch_tile_t3<FMT, D, NW, HPW, RT, true>(p, grid, stream)
-                                         : launch_tile_t3<FMT, D, NW, HPW, RT, false>(p, grid, stream);
+    return (p.a.page_tokens & 15u) == 0u ? launch_tile_t3<FMT, D, NW, HPW, RT, TS, true>(p, grid, stream)
+                                         : launch_tile_t3<FMT, D, NW, HPW, RT, TS, false>(p, grid, stream);
+}
+
+// Heads per workgroup of a two-part launch (TS == 2), 0 for one part.
+//
+// An implicit-tile launch has only tiles x kv_heads workgroups and no scratch
+// to split K over, and its waves are bound by instruction issue: 5-6 one-head
+// waves load two of the four SIMDs twice, and up to 256 workgroups leave the
+// rest of the chip idle. In two parts (waves on the even and the odd chunks of
+// each staged pair, joined in LDS) 6 heads put 3 waves on every SIMD; where the
+// tiles alone do not reach the 256 CUs the heads go to workgroups of 4 or 2.
+// Launcher times, one part -> two (us, 24/4 heads of 256; rows + context):
+//   FP8   48+0 12.5 -> 9.4 (2 heads)      BF16  128+1024 55.6 -> 42.8 (2)
+//   FP8   512+4096 166 -> 111 (4; 6: 122) PSQ4  512+4096 218 -> 172 (4; 6: 192)
+//   FP8   700+1024 69.3 -> 55.7 (6; 4: 81) PSQ8 1024+2048 157 -> 129 (6; 4: 207)
+//   FP8   2048+2048 262 -> 199 (6)        BF16  2048+0 154 -> 127 (6)
+// so the smallest workgroups that stay within one per CU win, then all heads.
+// A PSQ workgroup dequantizes for all its heads, so 2 of them pay only on a
+// nearly empty chip (8/1 heads of 128, PSQ8 128+1024: 4 heads 33.1, 2 34.9;
+// 48+0: 8.9 and 8.3). Beyond one workgroup per CU: 5-6 heads always (SIMD
+// balance), 1-2 heads (the other waves have no head), 3-4 and 7-8 only where
+// one CU holds one one-part workgroup anyway (BF16 at 256, 16/4 heads 2048+2048
+// 289 -> 247; PSQ8 16/2 heads of 128, 4096+0 246 -> 185); FP8 and PSQ at 256
+// would lose (16/4 heads 2048+2048: FP8 156 -> 171, PSQ4 249 -> 266). 16 waves
+// (7-8 heads) need 128 registers a wave: head_dim <= 128.
+uint32_t two_part_heads(const TileParams& p, bool psq, bool bf16, uint64_t tiles, uint32_t qpk) {
+    if (p.n_tiles != 0u || p.splits != 1u || p.partials != nullptr) return 0u;
+    constexpr uint64_t kCus = 256;
+    const uint64_t units = tiles * p.a.kv_heads;
+    if (qpk <= 2u || units * ((qpk + 1u) / 2u) <= (psq ? kCus / 4u : kCus)) return 2u;
+    if (units * ((qpk + 3u) / 4u) <= kCus) return 4u;
+    if (qpk == 5u || qpk == 6u) return 6u;
+    const bool wide = p.a.head_dim == 256u;
+    if (units > kCus && !(wide ? bf16 : psq && qpk > 4u)) return 0u;
+    return qpk <= 4u ? 4u : wide ? 0u : 8u;
 }
 
 // Waves and heads per wave by group size: up to 4 heads one per wave (4
@@ -1522,6 +1665,7 @@ hipError_t launch_tile_t2(const TileParams& p, uint64_t grid, hipStream_t stream
 // Grouped launches (tiles_per_group == kTileGroup, 1-8 heads): kTileGroup
 // waves, one per tile, each on two heads of the group's head part, so each
 // converted K/V fragment feeds two MFMAs; 2 waves on every SIMD.
+// Launches of implicit tiles run in two parts by two_part_heads.
 // Wave counts that load the SIMDs unevenly (3 waves per workgroup) lose: the
 // chunk barrier waits on the doubly loaded SIMDs. PSQ grouped launches go to
 // paged_tile_psq_group_kernel (the same workgroup shape on a shared f16
@@ -1531,8 +1675,10 @@ hipError_t launch_tile_t(const TileParams& p, hipStream_t stream) {
     const uint32_t qpk = p.a.q_heads / p.a.kv_heads;
     const uint64_t tiles = p.n_tiles != 0u ? p.n_tiles : (p.a.rows + kTileRows - 1) / kTileRows;
     const bool grouped = p.tiles_per_group == (uint32_t)kTileGroup && grouped_heads(qpk);
-    const uint64_t grid = grouped ? (tiles + kTileGroup - 1) / kTileGroup * ((qpk + 1u) / 2u) * p.a.kv_heads * p.splits
-                                  : tiles * p.a.kv_heads * p.splits;
+    const uint32_t wh = two_part_heads(p, fmt_psq<FMT>(), FMT == kFmtBf16, tiles, qpk);
+    const uint64_t grid = wh != 0u ? tiles * ((qpk + wh - 1u) / wh) * p.a.kv_heads
+                          : grouped ? (tiles + kTileGroup - 1) / kTileGroup * ((qpk + 1u) / 2u) * p.a.kv_heads * p.splits
+                                    : tiles * p.a.kv_heads * p.splits;
     if (grid == 0u || grid > 0x7FFFFFFFull) return hipErrorInvalidValue;
     if constexpr (fmt_psq<FMT>()) {
         // PSQ: one shared f16 dequantization per chunk, then f16 MFMAs
@@ -1542,10 +1688,22 @@ hipError_t launch_tile_t(const TileParams& p, hipStream_t stream) {
         // dequantization (5-6 heads: the reference's prefill launcher over
         // config 5's chunks 2.13 -> 1.87 ms PSQ4, 2.17 -> 1.95 ms PSQ8
         // against 6 waves with 4 dequantizing)
+        if (wh == 2u) return launch_tile_pg<FMT, D, 4, 1, 1, 2>(p, grid, stream);
+        if (wh == 4u) return launch_tile_pg<FMT, D, 8, 1, 1, 2>(p, grid, stream);
+        if (wh == 6u) return launch_tile_pg<FMT, D, 12, 1, 1, 2>(p, grid, stream);
+        if constexpr (D <= 128) {
+            if (wh == 8u) return launch_tile_pg<FMT, D, 16, 1, 1, 2>(p, grid, stream);
+        }
         if (qpk <= 4u) return launch_tile_pg<FMT, D, 4, 1, 1>(p, grid, stream);
         return launch_tile_pg<FMT, D, 8, 1, 1>(p, grid, stream);
     } else {
         if (grouped) return launch_tile_t2<FMT, D, kTileGroup, 2, kTileGroup>(p, grid, stream);
+        if (wh == 2u) return launch_tile_t2<FMT, D, 4, 1, 1, 2>(p, grid, stream);
+        if (wh == 4u) return launch_tile_t2<FMT, D, 8, 1, 1, 2>(p, grid, stream);
+        if (wh == 6u) return launch_tile_t2<FMT, D, 12, 1, 1, 2>(p, grid, stream);
+        if constexpr (D <= 128) {
+            if (wh == 8u) return launch_tile_t2<FMT, D, 16, 1, 1, 2>(p, grid, stream);
+        }
         if (qpk <= 4u) return launch_tile_t2<FMT, D, 4, 1>(p, grid, stream);
         if (qpk <= 6u) return launch_tile_t2<FMT, D, 6, 1>(p, grid, stream);
         return launch_tile_t2<FMT, D, 8, 1>(p, grid, stream);
