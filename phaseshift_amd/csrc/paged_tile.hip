@@ -234,7 +234,7 @@ template <int NW, int HPW, int RT, int TS>
 __device__ __forceinline__ bool tile_workgroup(const TileParams& p, uint32_t qpk, uint32_t& split,
                                                uint32_t& hpart, uint32_t& kv_head, uint32_t& group) {
     hpart = 0u;
-    if constexpr (RT == 1 && TS == 1) {
+    if constexpr (RT == 1) {
         const uint32_t count = p.n_tiles != 0u ? p.n_tiles : (p.a.rows + kTileRows - 1u) / kTileRows;
         if (p.splits > 1u && (uint64_t)count * p.splits <= kDenseTileUnits) {
             kv_head = blockIdx.x % p.a.kv_heads;
@@ -1643,8 +1643,20 @@ hipError_t launch_tile_t2(const TileParams& p, uint64_t grid, hipStream_t stream
 // 289 -> 247; PSQ8 16/2 heads of 128, 4096+0 246 -> 185); FP8 and PSQ at 256
 // would lose (16/4 heads 2048+2048: FP8 156 -> 171, PSQ4 249 -> 266). 16 waves
 // (7-8 heads) need 128 registers a wave: head_dim <= 128.
-uint32_t two_part_heads(const TileParams& p, bool psq, bool bf16, uint64_t tiles, uint32_t qpk) {
-    if (p.n_tiles != 0u || p.splits != 1u || p.partials != nullptr) return 0u;
+//
+// Explicit tiles and split launches (verify blocks) take two parts for 5-6
+// heads, unless a split's range is one part anyway. Whole verify calls (us,
+// 24/4 heads of 256): FP8 8 blocks of 16 rows over 2-16k tokens 55.4 -> 51.3, 32
+// over 2-8k 166 -> 154, 16 of 12 rows over 256-2000 tokens 77 -> 60; BF16 62.2
+// -> 59.1, 211 -> 205, 96 -> 80. PSQ gains less (PSQ4 32 blocks 209 -> 197) and
+// loses 2-2.5 us of 24-32 on ranges of 272 tokens: splits past 512 tokens only.
+uint32_t two_part_heads(const TileParams& p, bool grouped, bool psq, bool bf16, uint64_t tiles, uint32_t qpk) {
+    if (grouped) return 0u;
+    if (p.n_tiles != 0u || p.splits != 1u) {
+        const uint64_t range = (uint64_t)p.pages_per_split * p.a.page_tokens;
+        const bool two = p.splits > 1u ? range > (psq ? 2u : 1u) * kTwoPartTokens : !psq;
+        return (qpk == 5u || qpk == 6u) && two ? 6u : 0u;
+    }
     constexpr uint64_t kCus = 256;
     const uint64_t units = tiles * p.a.kv_heads;
     if (qpk <= 2u || units * ((qpk + 1u) / 2u) <= (psq ? kCus / 4u : kCus)) return 2u;
@@ -1675,8 +1687,8 @@ hipError_t launch_tile_t(const TileParams& p, hipStream_t stream) {
     const uint32_t qpk = p.a.q_heads / p.a.kv_heads;
     const uint64_t tiles = p.n_tiles != 0u ? p.n_tiles : (p.a.rows + kTileRows - 1) / kTileRows;
     const bool grouped = p.tiles_per_group == (uint32_t)kTileGroup && grouped_heads(qpk);
-    const uint32_t wh = two_part_heads(p, fmt_psq<FMT>(), FMT == kFmtBf16, tiles, qpk);
-    const uint64_t grid = wh != 0u ? tiles * ((qpk + wh - 1u) / wh) * p.a.kv_heads
+    const uint32_t wh = two_part_heads(p, grouped, fmt_psq<FMT>(), FMT == kFmtBf16, tiles, qpk);
+    const uint64_t grid = wh != 0u ? tiles * ((qpk + wh - 1u) / wh) * p.a.kv_heads * p.splits
                           : grouped ? (tiles + kTileGroup - 1) / kTileGroup * ((qpk + 1u) / 2u) * p.a.kv_heads * p.splits
                                     : tiles * p.a.kv_heads * p.splits;
     if (grid == 0u || grid > 0x7FFFFFFFull) return hipErrorInvalidValue;
