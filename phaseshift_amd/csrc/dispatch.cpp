@@ -288,13 +288,13 @@ DecodeSplit choose_tile_split(uint32_t n_tiles, uint32_t tiles_per_group, uint32
         // Ungrouped tiles split into dense (tile, split) units, dealt
         // longest first over the XCDs. Cost model, in pages: rounds of units
         // over the CUs x (pages per split + kTileSplitFixedPages of start-up:
-        // Q split, block-table window, partial write). One workgroup per CU:
-        // a 6-wave workgroup (5-6 heads) puts two waves on SIMDs 0 and 1, and
-        // a second one doubles those (measured on 8 verify blocks of config
-        // 5: 236 units of 80 pages 66 us, 280 units of 66 pages 102 us).
+        // Q split, block-table window, partial write). One workgroup per CU
+        // for 5-6 heads: the 12 waves of a two-part workgroup fill its SIMDs'
+        // registers (6 one-part waves put two on SIMDs 0 and 1, and a second
+        // workgroup doubled those: 8 verify blocks as 236 units of 80 pages 66
+        // us, as 280 of 66 pages 102 us).
         constexpr uint64_t kTileSplitFixedPages = 16;
-        // 5-6 heads: the 6-wave kernel (PSQ: 8 waves, 2 per SIMD, which fill the
-        // registers of a CU's SIMDs at 168 each)
+        // 5-6 heads: 12 waves, or 6 on short splits (PSQ: 8), at 168 registers each
         const bool nw6 = q_per_kv > 4u && q_per_kv <= 6u;
         const uint64_t slots =
             (uint64_t)device_cus() * (nw6 ? 1u : psk::tile_workgroups_per_cu(kv_dtype, head_dim, q_per_kv, false));

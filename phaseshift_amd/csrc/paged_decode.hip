@@ -98,9 +98,11 @@ __device__ __forceinline__ i16x4 lds_read_tr16(const uint8_t* p) {
 // Units of work of one row: splits that hold pages, 0 for a row the kernel
 // skips (invalid slot, position past the block table).
 __device__ __forceinline__ uint32_t row_units(const psk_paged_attention_args& a, uint32_t splits,
-                                              uint32_t pps, uint32_t r) {
-    if (a.row_sequence_slots[r] >= a.max_sequences) return 0u;
-    const uint64_t vis = (uint64_t)a.row_positions[r] + 1u;
+                                              uint32_t pps, uint32_t r, uint32_t& slot, uint32_t& pos) {
+    slot = a.row_sequence_slots[r];
+    pos = a.row_positions[r];
+    if (slot >= a.max_sequences) return 0u;
+    const uint64_t vis = (uint64_t)pos + 1u;
     if (vis > (uint64_t)a.block_table_stride * a.page_tokens || vis > 0xFFFFFFFFull) return 0u;
     const uint32_t pc = ((uint32_t)vis + a.page_tokens - 1u) / a.page_tokens;
     const uint32_t per = split_pages(pc, splits, pps);
@@ -117,22 +119,32 @@ constexpr uint64_t kDenseDecodeUnits = 4096;
 // last, row-major, then the last split of every row). Unsplit launches: unit
 // u is row u. Larger split launches: unit u is (u / splits, u % splits).
 // Returns false for a unit without work. All NW*64 threads of the workgroup
-// must call it (the branch taken is uniform).
+// must call it (the branch taken is uniform). slot, pos: the row's.
 template <int NW>
 __device__ bool find_unit(const psk_paged_attention_args& a, uint32_t splits, uint32_t pps,
-                          uint32_t unit, uint32_t& row, uint32_t& split) {
+                          uint32_t unit, uint32_t& row, uint32_t& split, uint32_t& slot, uint32_t& pos) {
     if (splits == 1u) {
         row = unit;
         split = 0u;
-        return unit < a.rows && row_units(a, 1u, pps, unit) != 0u;
+        return unit < a.rows && row_units(a, 1u, pps, unit, slot, pos) != 0u;
     }
     if ((uint64_t)a.rows * splits > kDenseDecodeUnits) {
         row = unit / splits;
         split = unit % splits;
-        return row < a.rows && split < row_units(a, splits, pps, row);
+        return row < a.rows && split < row_units(a, splits, pps, row, slot, pos);
     }
-    return find_dense_unit<NW>(
-        a.rows, [&](uint32_t r) { return row_units(a, splits, pps, r); }, unit, row, split);
+    uint32_t s = 0u, q = 0u;   // of the last row this thread looked at
+    auto units = [&](uint32_t r) { return row_units(a, splits, pps, r, s, q); };
+    if (a.rows <= kWaveItems) {
+        if (!find_dense_unit_wave(a.rows, units, unit, row, split)) return false;
+        slot = __builtin_amdgcn_readlane(s, row);
+        pos = __builtin_amdgcn_readlane(q, row);
+        return true;
+    }
+    if (!find_dense_unit<NW>(a.rows, units, unit, row, split)) return false;
+    slot = a.row_sequence_slots[row];
+    pos = a.row_positions[row];
+    return true;
 }
 
 constexpr uint32_t kPageWindow = 1024;   // block-table entries staged in LDS per pass
@@ -215,11 +227,10 @@ __global__ __launch_bounds__(NW * 64, waves_per_simd<FMT>()) void paged_decode_k
     // blockIdx = unit * G + sub: G independent kv-head groups or G kv heads
     const uint32_t G = kIndep ? (a.kv_heads + NW - 1u) / NW : a.kv_heads;
     const uint32_t sub = blockIdx.x % G;
-    uint32_t row, split;
-    if (!find_unit<NW>(a, splits, p.pages_per_split, blockIdx.x / G, row, split)) return;
+    uint32_t row, split, slot, pos;
+    if (!find_unit<NW>(a, splits, p.pages_per_split, blockIdx.x / G, row, split, slot, pos)) return;
     const uint32_t kv_head = kIndep ? sub * NW + wave : sub;
-    const uint32_t slot = a.row_sequence_slots[row];
-    const uint32_t visible = a.row_positions[row] + 1u;
+    const uint32_t visible = pos + 1u;
     const uint32_t P = a.page_tokens;
     const uint32_t pc = (visible + P - 1u) / P;
     const uint32_t per = split_pages(pc, splits, p.pages_per_split);
@@ -227,6 +238,8 @@ __global__ __launch_bounds__(NW * 64, waves_per_simd<FMT>()) void paged_decode_k
     const uint32_t pe = (split == splits - 1u) ? pc : min(pc, pb + per);
     const uint32_t t_end = min(pe * P, visible);
     const uint32_t* bt = a.block_tables + (uint64_t)slot * a.block_table_stride;
+    // this thread's entry of the first window, on its way while Q is prepared
+    const uint32_t bt_first = pb + tid < pe ? bt[pb + tid] : 0u;
     // Everything above is uniform over the workgroup (row, split), so every
     // wave reaches the barriers below; an independent wave past the last kv
     // head only helps stage the block table.
@@ -402,7 +415,8 @@ __global__ __launch_bounds__(NW * 64, waves_per_simd<FMT>()) void paged_decode_k
     for (uint32_t wp = pb; wp < pe; wp += kWin) {
         const uint32_t wp_end = min(pe, wp + kWin);
         __syncthreads();
-        for (uint32_t i = tid; i < wp_end - wp; i += NT) win[i] = bt[wp + i];
+        if (wp == pb && tid < wp_end - wp) win[tid] = bt_first;
+        for (uint32_t i = wp == pb ? tid + NT : tid; i < wp_end - wp; i += NT) win[i] = bt[wp + i];
         __syncthreads();
         const uint32_t ts = wp * P;
         const uint32_t te = min(wp_end * P, t_end);

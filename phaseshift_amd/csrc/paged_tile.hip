@@ -172,7 +172,9 @@ constexpr int tile_waves_per_simd(int hpw, int nw = 0) { return nw > 12 ? 4 : hp
 constexpr bool grouped_heads(uint32_t q_per_kv) { return q_per_kv >= 1u && q_per_kv <= 8u; }
 
 // RT: row tiles per workgroup. RT == 1: the NW waves split the GQA group's
-// heads (HPW each) of one tile. RT > 1 (NW == RT): wave w owns tile w of a
+// heads (HPW each) of one tile; TS == 2: two waves per head, on the even and
+// the odd chunks of each staged pair, NW / 2 heads of the head part (blockIdx),
+// see two_part_heads. RT > 1 (NW == RT): wave w owns tile w of a
 // group of RT consecutive tiles of one sequence and HPW heads of the group's
 // head part (blockIdx); the tiles share every staged K/V chunk.
 // Split units of ungrouped tile t: the splits of its visible range that hold
@@ -194,8 +196,6 @@ __device__ uint32_t tile_units(const TileParams& p, uint32_t t) {
     if (r0 >= a.rows) return 0u;
     nrows = min(nrows, a.rows - r0);
     if (nrows == 0u) return 0u;
-    const uint32_t slot = a.row_sequence_slots[r0];
-    if (slot >= a.max_sequences) return 0u;
     const uint64_t cap = (uint64_t)a.block_table_stride * a.page_tokens;
     // all rows' loads first (rows past the tile repeat its last row)
     uint32_t sl[kTileRows], ps[kTileRows];
@@ -205,6 +205,8 @@ __device__ uint32_t tile_units(const TileParams& p, uint32_t t) {
         sl[j] = a.row_sequence_slots[r];
         ps[j] = a.row_positions[r];
     }
+    const uint32_t slot = sl[0];
+    if (slot >= a.max_sequences) return 0u;
     uint32_t vis_max = 0u;
 #pragma unroll
     for (int j = 0; j < kTileRows; ++j) {
