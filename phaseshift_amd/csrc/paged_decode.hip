@@ -35,6 +35,7 @@
 // single bf16 operand (8 significant bits) in the PV product; BF16 and FP8
 // carry P as a bf16 hi + lo pair instead.
 #include "device_common.h"
+#include "split_units.h"
 
 #include <phaseshift_kv/paged_attention.h>
 
@@ -61,10 +62,6 @@ constexpr int kWaves = 4;
 constexpr int kMaxQPerKV = 16;
 constexpr uint32_t kMaxSplits = 1024;
 using ps::kernel::kPagedAttentionHeadLimit;
-
-__device__ __forceinline__ uint32_t split_pages(uint32_t pc, uint32_t splits, uint32_t pps) {
-    return pps != 0u ? pps : (pc + splits - 1u) / splits;
-}
 
 // Loads 8 bf16 of a query head as an MFMA operand (zeros past the group).
 __device__ __forceinline__ bf16x8 load_q8(const uint16_t* q, bool ok) {
@@ -95,18 +92,14 @@ __device__ __forceinline__ i16x4 lds_read_tr16(const uint8_t* p) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(p));
 }
 
-// Units of work of one row: splits that hold pages, 0 for a row the kernel
-// skips (invalid slot, position past the block table).
+// Units of work of one row: splits that hold pages, 0 for a row the kernels
+// skip (invalid slot, position past the block table or the 32-bit range).
 __device__ __forceinline__ uint32_t row_units(const psk_paged_attention_args& a, uint32_t splits,
                                               uint32_t pps, uint32_t r, uint32_t& slot, uint32_t& pos) {
     slot = a.row_sequence_slots[r];
     pos = a.row_positions[r];
     if (slot >= a.max_sequences) return 0u;
-    const uint64_t vis = (uint64_t)pos + 1u;
-    if (vis > (uint64_t)a.block_table_stride * a.page_tokens || vis > 0xFFFFFFFFull) return 0u;
-    const uint32_t pc = ((uint32_t)vis + a.page_tokens - 1u) / a.page_tokens;
-    const uint32_t per = split_pages(pc, splits, pps);
-    return min(splits, (pc + per - 1u) / per);
+    return used_splits(pos, (uint64_t)a.block_table_stride * a.page_tokens, a.page_tokens, splits, pps);
 }
 
 // Largest rows x splits of a split launch whose workgroups take dense units:
@@ -938,13 +931,9 @@ __global__ __launch_bounds__(kThreads) void split_reduce_kernel(const DecodePara
     const uint32_t kv_head = (blockIdx.x / qpk) % a.kv_heads;
     const uint32_t row = blockIdx.x / (qpk * a.kv_heads);
     if (row >= a.rows) return;
-    const uint32_t slot = a.row_sequence_slots[row];
-    const uint64_t vis64 = (uint64_t)a.row_positions[row] + 1u;
-    if (slot >= a.max_sequences) return;
-    if (vis64 > (uint64_t)a.block_table_stride * a.page_tokens) return;
-    const uint32_t pc = ((uint32_t)vis64 + a.page_tokens - 1u) / a.page_tokens;
-    const uint32_t per = split_pages(pc, p.splits, p.pages_per_split);
-    const uint32_t n_used = min(p.splits, (pc + per - 1u) / per);
+    uint32_t slot, pos;
+    const uint32_t n_used = row_units(a, p.splits, p.pages_per_split, row, slot, pos);
+    if (n_used == 0u) return;   // the clamps below need one split
     const uint32_t stride = qpk * (2u + kPagedAttentionHeadLimit);
     const float* base = p.partials + (uint64_t)(row * a.kv_heads + kv_head) * p.splits * stride;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;

@@ -17,6 +17,7 @@
 // split-K writes the decode kernel's partial layout and the same combine
 // kernel finishes it.
 #include "device_common.h"
+#include "split_units.h"
 
 #include <type_traits>
 
@@ -215,8 +216,7 @@ __device__ uint32_t tile_units(const TileParams& p, uint32_t t) {
     }
     if (vis_max == 0u) return 0u;
     const uint32_t pc = (vis_max + a.page_tokens - 1u) / a.page_tokens;
-    const uint32_t per = p.pages_per_split != 0u ? p.pages_per_split : (pc + p.splits - 1u) / p.splits;
-    return min(p.splits, (pc + per - 1u) / per);
+    return splits_of_pages(pc, p.splits, p.pages_per_split);
 }
 
 // Largest tiles x splits of a launch whose workgroups take dense units: each

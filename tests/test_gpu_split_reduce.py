@@ -101,3 +101,35 @@ def test_split_reduce_nan_split_and_invalid_slot_leave_rows_unwritten(dev):
         w = want[2, hh * D:(hh + 1) * D]
         np.testing.assert_allclose(got[2, hh * D:(hh + 1) * D], w, rtol=2e-5, atol=2e-5 * np.abs(w).max())
     assert np.all(got[3] == 7.0)
+
+
+def test_split_reduce_leaves_rows_without_splits_unwritten(dev):
+    """A table of 65536 pages of 65536 tokens holds every 32-bit position, but
+    the last page below 2^32 has no page count in 32 bits: no split of such a
+    row holds partials, and the combine leaves it unwritten, as the attention
+    kernels skip it."""
+    splits, page, pps, qh, kvh, D = 4, 65536, 16384, 4, 2, 256
+    vis = [1, 2**32, 2**32 - page + 1, 2**32 - page, 2**31]
+    used = np.array([1, 0, 0, 4, 2], np.uint32)
+    rows, qpk = len(vis), qh // kvh
+    rng = np.random.default_rng(5)
+    part = np.empty((rows, kvh, splits, qpk * (2 + HEAD_LIMIT)), np.float32)
+    part[..., :qpk] = rng.uniform(-3.0, 3.0, (rows, kvh, splits, qpk))
+    part[..., qpk:2 * qpk] = rng.uniform(0.5, 4.0, (rows, kvh, splits, qpk))
+    part[..., 2 * qpk:] = rng.standard_normal((rows, kvh, splits, qpk * HEAD_LIMIT))
+    g = ops.PoolGeometry(1, 1, page, kvh, D)
+    q = torch.zeros((rows, qh * D), dtype=torch.bfloat16, device=dev)
+    out = torch.full((rows, qh * D), 7.0, dtype=torch.float32, device=dev)
+    a = ops.attention_args(g, 0, q, out, to_dev(np.zeros(rows, np.uint32)),
+                           to_dev((np.array(vis, np.uint64) - 1).astype(np.uint32)),
+                           to_dev(np.zeros((1, 65536), np.uint32)), qh)
+    parts = torch.from_numpy(part).to(dev)
+    P.check("reduce", P.lib().psk_attention_paged_split_reduce_ex(
+        C.byref(a), parts.data_ptr(), splits, pps, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    geom = dict(q_heads=qh, kv_heads=kvh, head_dim=D, max_sequences=1)
+    keep = np.nonzero(used)[0]
+    want = oracle.split_reduce(geom, part[keep], splits, used[keep], np.zeros(len(keep), np.uint32), len(keep))
+    np.testing.assert_allclose(got[keep], want, rtol=2e-5, atol=2e-5 * np.abs(want).max())
+    assert np.all(got[used == 0] == 7.0)
