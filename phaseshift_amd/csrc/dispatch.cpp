@@ -22,19 +22,39 @@ uint32_t tile_workgroups_per_cu(uint32_t kv_dtype, uint32_t head_dim, uint32_t q
 hipError_t launch_paged_tiles(const psk_paged_attention_args& a, uint32_t kv_dtype, const void* k,
                               const void* v, const void* ks, const void* vs,
                               const uint32_t* tile_begin, const uint32_t* tile_rows,
-                              uint32_t n_tiles, uint32_t tiles_per_group, float* partials,
-                              uint32_t splits, uint32_t pages_per_split, hipStream_t stream);
+                              uint32_t n_tiles, uint32_t tiles_per_group, uint32_t part_heads,
+                              float* partials, uint32_t splits, uint32_t pages_per_split,
+                              hipStream_t stream);
+uint32_t tile_part_heads(const psk_paged_attention_args& a, uint32_t kv_dtype, bool split, uint64_t range,
+                         uint64_t units);
 uint32_t tile_group_size(uint32_t q_per_kv, uint32_t kv_dtype);
 uint32_t tile_dense_units_limit();
 uint64_t tile_launch_workgroups(uint64_t n_tiles, uint32_t tiles_per_group, uint32_t q_per_kv,
                                 uint32_t kv_heads);
 bool paged_tiles_supported(const psk_paged_attention_args& a, uint32_t kv_dtype, const void* k,
                            const void* v, const void* ks, const void* vs);
+
+// CUs of the device (256 on an MI355X, and where there is none).
+uint32_t device_cus() {
+    static const uint32_t cus = [] {
+        int dev = 0;
+        hipDeviceProp_t prop{};
+        if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess ||
+            prop.multiProcessorCount <= 0) {
+            (void)hipGetLastError();
+            return 256u;   // MI355X
+        }
+        return static_cast<uint32_t>(prop.multiProcessorCount);
+    }();
+    return cus;
+}
+
 }  // namespace psk
 
 namespace ps::qwen35::runtime {
 
 using ::ps::kernel::PagedAttentionCommonArgs;
+using ::psk::device_cus;
 using ::ps::kernel::PagedAttentionOutputDType;
 
 namespace {
@@ -58,20 +78,6 @@ namespace {
 // MI355X geometry the chooser models: workgroups are dealt round-robin to 8
 // XCDs (block b runs on XCD b mod 8), each with multiProcessorCount/8 CUs.
 constexpr uint32_t kXcds = 8;
-
-uint32_t device_cus() {
-    static const uint32_t cus = [] {
-        int dev = 0;
-        hipDeviceProp_t prop{};
-        if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess ||
-            prop.multiProcessorCount <= 0) {
-            (void)hipGetLastError();
-            return 256u;   // MI355X
-        }
-        return static_cast<uint32_t>(prop.multiProcessorCount);
-    }();
-    return cus;
-}
 
 // Makespan (seconds) of the decode kernel's units (dense, longest first, unit
 // u on XCD u mod 8, given in bytes) under greedy dispatch onto `slots`
@@ -489,6 +495,18 @@ Status plan_paged_attention_step(const PagedAttentionStep& step, PagedAttentionP
             step.max_visible_tokens, pbytes, tile_vis);
         k.splits = s.splits;
         k.pages_per_split = s.pages_per_split;
+        if (group == 1u && c.kv_heads != 0 && c.page_tokens != 0) {
+            uint64_t units = 0, range = 0;
+            for (uint32_t vis : tile_vis) {
+                const uint64_t pages = ((uint64_t)vis + c.page_tokens - 1u) / c.page_tokens;
+                units += s.splits > 1u ? (pages + s.pages_per_split - 1u) / s.pages_per_split : 1u;
+                range = std::max<uint64_t>(range, vis);
+            }
+            if (s.splits > 1u) range = std::min(range, (uint64_t)s.pages_per_split * c.page_tokens);
+            k.part_heads = psk::tile_part_heads(reinterpret_cast<const psk_paged_attention_args&>(c),
+                                                static_cast<uint32_t>(step.kv_dtype), s.splits > 1u, range,
+                                                units * c.kv_heads);
+        }
         Status st = push(k);
         if (!st.ok()) return st;
     }
@@ -616,7 +634,7 @@ hipError_t launch_paged_attention_plan(const PagedAttentionStep& step, const Pag
                                            step.v_scale_pool)) {
                 e = psk::launch_paged_tiles(*ca, kvd, step.k_pool, step.v_pool, step.k_scale_pool,
                                             step.v_scale_pool, tb.data(), tr.data(), k.tile_count,
-                                            k.tiles_per_group, parts, k.splits,
+                                            k.tiles_per_group, k.part_heads, parts, k.splits,
                                             k.pages_per_split, stream);
                 // one combine per run of adjacent requests of the launch (rows of
                 // other requests inside the launch's region hold no partials)

@@ -18,12 +18,16 @@
 // kernel finishes it.
 #include "device_common.h"
 #include "split_units.h"
+#include "tile_parts.h"
 
 #include <type_traits>
 
 #include <phaseshift_kv/paged_attention.h>
 
 namespace psk {
+
+uint32_t device_cus();   // dispatch.cpp
+
 namespace {
 
 using ps::kernel::kPagedAttentionHeadLimit;
@@ -141,12 +145,6 @@ __device__ __forceinline__ float q_split_e4m3(const uint16_t* qrow, bool ok, uin
     return __builtin_ldexpf(1.0f, -sh);
 }
 
-// A two-part launch's tiles of up to this many tokens run as one part: joining
-// the parts costs 1-2 us, about what splitting 8 chunks gains (FP8, 24/4 heads,
-// 6 per workgroup, 128 rows without context 15.1 us, in two parts 16.3; 512
-// rows 29.6 and 27.2).
-constexpr uint32_t kTwoPartTokens = 256;
-
 constexpr uint32_t kTilePageWindow = 1024;   // block-table entries staged in LDS per pass
 
 // LDS bytes of one pipeline stage: K and V of a 32-token chunk (lane-major DMA
@@ -175,7 +173,7 @@ constexpr bool grouped_heads(uint32_t q_per_kv) { return q_per_kv >= 1u && q_per
 // RT: row tiles per workgroup. RT == 1: the NW waves split the GQA group's
 // heads (HPW each) of one tile; TS == 2: two waves per head, on the even and
 // the odd chunks of each staged pair, NW / 2 heads of the head part (blockIdx),
-// see two_part_heads. RT > 1 (NW == RT): wave w owns tile w of a
+// see tile_parts.h. RT > 1 (NW == RT): wave w owns tile w of a
 // group of RT consecutive tiles of one sequence and HPW heads of the group's
 // head part (blockIdx); the tiles share every staged K/V chunk.
 // Split units of ungrouped tile t: the splits of its visible range that hold
@@ -1623,52 +1621,6 @@ hipError_t launch_tile_t2(const TileParams& p, uint64_t grid, hipStream_t stream
                                          : launch_tile_t3<FMT, D, NW, HPW, RT, TS, false>(p, grid, stream);
 }
 
-// Heads per workgroup of a two-part launch (TS == 2), 0 for one part.
-//
-// An implicit-tile launch has only tiles x kv_heads workgroups and no scratch
-// to split K over, and its waves are bound by instruction issue: 5-6 one-head
-// waves load two of the four SIMDs twice, and up to 256 workgroups leave the
-// rest of the chip idle. In two parts (waves on the even and the odd chunks of
-// each staged pair, joined in LDS) 6 heads put 3 waves on every SIMD; where the
-// tiles alone do not reach the 256 CUs the heads go to workgroups of 4 or 2.
-// Launcher times, one part -> two (us, 24/4 heads of 256; rows + context):
-//   FP8   48+0 12.5 -> 9.4 (2 heads)      BF16  128+1024 55.6 -> 42.8 (2)
-//   FP8   512+4096 166 -> 111 (4; 6: 122) PSQ4  512+4096 218 -> 172 (4; 6: 192)
-//   FP8   700+1024 69.3 -> 55.7 (6; 4: 81) PSQ8 1024+2048 157 -> 129 (6; 4: 207)
-//   FP8   2048+2048 262 -> 199 (6)        BF16  2048+0 154 -> 127 (6)
-// so the smallest workgroups that stay within one per CU win, then all heads.
-// A PSQ workgroup dequantizes for all its heads, so 2 of them pay only on a
-// nearly empty chip (8/1 heads of 128, PSQ8 128+1024: 4 heads 33.1, 2 34.9;
-// 48+0: 8.9 and 8.3). Beyond one workgroup per CU: 5-6 heads always (SIMD
-// balance), 1-2 heads (the other waves have no head), 3-4 and 7-8 only where
-// one CU holds one one-part workgroup anyway (BF16 at 256, 16/4 heads 2048+2048
-// 289 -> 247; PSQ8 16/2 heads of 128, 4096+0 246 -> 185); FP8 and PSQ at 256
-// would lose (16/4 heads 2048+2048: FP8 156 -> 171, PSQ4 249 -> 266). 16 waves
-// (7-8 heads) need 128 registers a wave: head_dim <= 128.
-//
-// Explicit tiles and split launches (verify blocks) take two parts for 5-6
-// heads, unless a split's range is one part anyway. Whole verify calls (us,
-// 24/4 heads of 256): FP8 8 blocks of 16 rows over 2-16k tokens 55.4 -> 51.3, 32
-// over 2-8k 166 -> 154, 16 of 12 rows over 256-2000 tokens 77 -> 60; BF16 62.2
-// -> 59.1, 211 -> 205, 96 -> 80. PSQ gains less (PSQ4 32 blocks 209 -> 197) and
-// loses 2-2.5 us of 24-32 on ranges of 272 tokens: splits past 512 tokens only.
-uint32_t two_part_heads(const TileParams& p, bool grouped, bool psq, bool bf16, uint64_t tiles, uint32_t qpk) {
-    if (grouped) return 0u;
-    if (p.n_tiles != 0u || p.splits != 1u) {
-        const uint64_t range = (uint64_t)p.pages_per_split * p.a.page_tokens;
-        const bool two = p.splits > 1u ? range > (psq ? 2u : 1u) * kTwoPartTokens : !psq;
-        return (qpk == 5u || qpk == 6u) && two ? 6u : 0u;
-    }
-    constexpr uint64_t kCus = 256;
-    const uint64_t units = tiles * p.a.kv_heads;
-    if (qpk <= 2u || units * ((qpk + 1u) / 2u) <= (psq ? kCus / 4u : kCus)) return 2u;
-    if (units * ((qpk + 3u) / 4u) <= kCus) return 4u;
-    if (qpk == 5u || qpk == 6u) return 6u;
-    const bool wide = p.a.head_dim == 256u;
-    if (units > kCus && !(wide ? bf16 : psq && qpk > 4u)) return 0u;
-    return qpk <= 4u ? 4u : wide ? 0u : 8u;
-}
-
 // Waves and heads per wave by group size: up to 4 heads one per wave (4
 // waves, so every SIMD issues part of the DMAs); 5-6 heads one per wave (6
 // waves: two workgroups put 3 waves on every SIMD); 7-8 heads one per wave
@@ -1679,17 +1631,16 @@ uint32_t two_part_heads(const TileParams& p, bool grouped, bool psq, bool bf16, 
 // Grouped launches (tiles_per_group == kTileGroup, 1-8 heads): kTileGroup
 // waves, one per tile, each on two heads of the group's head part, so each
 // converted K/V fragment feeds two MFMAs; 2 waves on every SIMD.
-// Launches of implicit tiles run in two parts by two_part_heads.
+// Launches in two parts (wh heads per workgroup, tile_parts.h) take 2 wh waves.
 // Wave counts that load the SIMDs unevenly (3 waves per workgroup) lose: the
 // chunk barrier waits on the doubly loaded SIMDs. PSQ grouped launches go to
 // paged_tile_psq_group_kernel (the same workgroup shape on a shared f16
 // dequantization of each chunk).
 template <int FMT, int D>
-hipError_t launch_tile_t(const TileParams& p, hipStream_t stream) {
+hipError_t launch_tile_t(const TileParams& p, uint32_t wh, hipStream_t stream) {
     const uint32_t qpk = p.a.q_heads / p.a.kv_heads;
     const uint64_t tiles = p.n_tiles != 0u ? p.n_tiles : (p.a.rows + kTileRows - 1) / kTileRows;
     const bool grouped = p.tiles_per_group == (uint32_t)kTileGroup && grouped_heads(qpk);
-    const uint32_t wh = two_part_heads(p, grouped, fmt_psq<FMT>(), FMT == kFmtBf16, tiles, qpk);
     const uint64_t grid = wh != 0u ? tiles * ((qpk + wh - 1u) / wh) * p.a.kv_heads * p.splits
                           : grouped ? (tiles + kTileGroup - 1) / kTileGroup * ((qpk + 1u) / 2u) * p.a.kv_heads * p.splits
                                     : tiles * p.a.kv_heads * p.splits;
@@ -1725,27 +1676,28 @@ hipError_t launch_tile_t(const TileParams& p, hipStream_t stream) {
 }
 
 template <int FMT>
-hipError_t launch_tile(const TileParams& p, hipStream_t stream) {
+hipError_t launch_tile(const TileParams& p, uint32_t wh, hipStream_t stream) {
     switch (p.a.head_dim) {
-        case 256: return launch_tile_t<FMT, 256>(p, stream);
-        case 128: return launch_tile_t<FMT, 128>(p, stream);
+        case 256: return launch_tile_t<FMT, 256>(p, wh, stream);
+        case 128: return launch_tile_t<FMT, 128>(p, wh, stream);
         case 64:
-            if constexpr (!fmt_psq<FMT>()) return launch_tile_t<FMT, 64>(p, stream);
+            if constexpr (!fmt_psq<FMT>()) return launch_tile_t<FMT, 64>(p, wh, stream);
             return hipErrorNotSupported;
         case 32:
-            if constexpr (FMT == kFmtBf16) return launch_tile_t<kFmtBf16, 32>(p, stream);
+            if constexpr (FMT == kFmtBf16) return launch_tile_t<kFmtBf16, 32>(p, wh, stream);
             return hipErrorNotSupported;
         default: return hipErrorNotSupported;
     }
 }
 
-// kv_dtype: PSK_KV_*; checked by the callers
-hipError_t launch_tile_fmt(const TileParams& p, uint32_t kv_dtype, hipStream_t stream) {
+// kv_dtype: PSK_KV_*; checked by the callers. wh: heads per workgroup in two
+// parts (tile_parts.h), 0 for one part
+hipError_t launch_tile_fmt(const TileParams& p, uint32_t kv_dtype, uint32_t wh, hipStream_t stream) {
     switch (kv_dtype) {
-        case PSK_KV_BF16: return launch_tile<kFmtBf16>(p, stream);
-        case PSK_KV_FP8_E4M3: return launch_tile<kFmtFp8>(p, stream);
-        case PSK_KV_PSQ8_W32: return launch_tile<kFmtPsq8>(p, stream);
-        case PSK_KV_PSQ4_W32: return launch_tile<kFmtPsq4>(p, stream);
+        case PSK_KV_BF16: return launch_tile<kFmtBf16>(p, wh, stream);
+        case PSK_KV_FP8_E4M3: return launch_tile<kFmtFp8>(p, wh, stream);
+        case PSK_KV_PSQ8_W32: return launch_tile<kFmtPsq8>(p, wh, stream);
+        case PSK_KV_PSQ4_W32: return launch_tile<kFmtPsq4>(p, wh, stream);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1793,17 +1745,36 @@ TileParams make_tile(const psk_paged_attention_args& c, const void* k, const voi
     return p;
 }
 
+TileShape tile_shape(const psk_paged_attention_args& c, uint32_t kv_dtype) {
+    return TileShape{c.head_dim, c.q_heads / c.kv_heads, c.kv_heads,
+                     kv_dtype == PSK_KV_PSQ4_W32 || kv_dtype == PSK_KV_PSQ8_W32, kv_dtype == PSK_KV_BF16};
+}
+
+// The prefill launchers: implicit tiles, unsplit.
+hipError_t launch_implicit_tiles(const TileParams& p, uint32_t kv_dtype, hipStream_t stream) {
+    return launch_tile_fmt(p, kv_dtype, implicit_part_heads(tile_shape(p.a, kv_dtype), p.a.rows, device_cus()), stream);
+}
+
 }  // namespace
+
+// Heads per workgroup in two parts of the step planner's launch of ungrouped
+// tiles, 0 for one part (explicit_part_heads).
+uint32_t tile_part_heads(const psk_paged_attention_args& a, uint32_t kv_dtype, bool split, uint64_t range,
+                         uint64_t units) {
+    return explicit_part_heads(tile_shape(a, kv_dtype), split, range, units, device_cus());
+}
 
 // Tile launch over explicit tiles (row_begin, rows) of one launch, any
 // number of them (chunks of kInlineTiles per launch). Used by the step
-// planner; every tile's rows must belong to one sequence.
+// planner; every tile's rows must belong to one sequence. part_heads:
+// tile_part_heads of an ungrouped launch.
 // ks / vs: FP8 f32 scale pools, PSQ bf16 block-scale pools, BF16 unused.
 hipError_t launch_paged_tiles(const psk_paged_attention_args& a, uint32_t kv_dtype, const void* k,
                               const void* v, const void* ks, const void* vs,
                               const uint32_t* tile_begin, const uint32_t* tile_rows,
-                              uint32_t n_tiles, uint32_t tiles_per_group, float* partials,
-                              uint32_t splits, uint32_t pages_per_split, hipStream_t stream) {
+                              uint32_t n_tiles, uint32_t tiles_per_group, uint32_t part_heads,
+                              float* partials, uint32_t splits, uint32_t pages_per_split,
+                              hipStream_t stream) {
     const hipError_t e = tile_validate(&a, k, v);
     if (e != hipSuccess) return e;
     if (!known_kv(kv_dtype)) return hipErrorInvalidValue;
@@ -1825,7 +1796,7 @@ hipError_t launch_paged_tiles(const psk_paged_attention_args& a, uint32_t kv_dty
             p.tile_begin[i] = tile_begin[b + i];
             p.tile_rows[i] = static_cast<uint8_t>(tile_rows[b + i]);
         }
-        const hipError_t le = launch_tile_fmt(p, kv_dtype, stream);
+        const hipError_t le = launch_tile_fmt(p, kv_dtype, tiles_per_group == 1u ? part_heads : 0u, stream);
         if (le != hipSuccess) return le;
     }
     return hipSuccess;
@@ -1892,9 +1863,9 @@ bool launch_prefill_psq_tiles(const psk_paged_attention_args& a, uint32_t kv_dty
                               const void* vc, const void* ks, const void* vs, hipStream_t stream,
                               hipError_t& err) {
     if (!paged_tiles_supported(a, kv_dtype, kc, vc, ks, vs)) return false;
-    err = launch_tile_fmt(make_tile(a, kc, vc, static_cast<const float*>(ks), static_cast<const float*>(vs),
-                                    nullptr, 1u, 0u),
-                          kv_dtype, stream);
+    err = launch_implicit_tiles(make_tile(a, kc, vc, static_cast<const float*>(ks), static_cast<const float*>(vs),
+                                          nullptr, 1u, 0u),
+                                kv_dtype, stream);
     return true;
 }
 
@@ -1910,8 +1881,8 @@ extern "C" int psk_attention_paged_prefill_bf16(const psk_paged_attention_args* 
     if (e != hipSuccess) return e;
     if (!psk::tile_shape_ok(*a, PSK_KV_BF16, k_pool, v_pool))
         return psk_attention_paged_bf16(a, k_pool, v_pool, stream);
-    return psk::launch_tile<psk::kFmtBf16>(
-        psk::make_tile(*a, k_pool, v_pool, nullptr, nullptr, nullptr, 1u, 0u), static_cast<hipStream_t>(stream));
+    return psk::launch_implicit_tiles(psk::make_tile(*a, k_pool, v_pool, nullptr, nullptr, nullptr, 1u, 0u),
+                                      PSK_KV_BF16, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int psk_attention_paged_prefill_fp8_e4m3(const psk_paged_attention_args* a,
@@ -1923,8 +1894,8 @@ extern "C" int psk_attention_paged_prefill_fp8_e4m3(const psk_paged_attention_ar
     if (k_scale_pool == nullptr || v_scale_pool == nullptr) return hipErrorInvalidValue;
     if (!psk::tile_shape_ok(*a, PSK_KV_FP8_E4M3, k_pool, v_pool))
         return psk_attention_paged_fp8_e4m3(a, k_pool, v_pool, k_scale_pool, v_scale_pool, stream);
-    return psk::launch_tile<psk::kFmtFp8>(
-        psk::make_tile(*a, k_pool, v_pool, k_scale_pool, v_scale_pool, nullptr, 1u, 0u),
+    return psk::launch_implicit_tiles(
+        psk::make_tile(*a, k_pool, v_pool, k_scale_pool, v_scale_pool, nullptr, 1u, 0u), PSK_KV_FP8_E4M3,
         static_cast<hipStream_t>(stream));
 }
 
@@ -1945,5 +1916,10 @@ extern "C" int psk_attention_paged_tile_split(const psk_paged_attention_args* a,
     const psk::TileParams p =
         psk::make_tile(*a, k_pool, v_pool, static_cast<const float*>(k_scale_pool),
                        static_cast<const float*>(v_scale_pool), partials, splits, pages_per_split);
-    return psk::launch_tile_fmt(p, kv_dtype, static_cast<hipStream_t>(stream));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (splits == 1u) return psk::launch_implicit_tiles(p, kv_dtype, st);
+    const uint64_t units = ((uint64_t)a->rows + psk::kTileRows - 1u) / psk::kTileRows * a->kv_heads * splits;
+    return psk::launch_tile_fmt(
+        p, kv_dtype,
+        psk::tile_part_heads(*a, kv_dtype, true, (uint64_t)pages_per_split * a->page_tokens, units), st);
 }

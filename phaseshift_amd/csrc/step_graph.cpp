@@ -37,7 +37,7 @@ void put(std::vector<uint8_t>& k, const T& v) {
 
 std::vector<uint8_t> plan_signature_bytes(const PagedAttentionStep& step, const PagedAttentionPlan& plan) {
     std::vector<uint8_t> k;
-    k.reserve(256 + plan.count * 40 + plan.tiles.size() * 8 + plan.combine.size() * 16);
+    k.reserve(256 + plan.count * 44 + plan.tiles.size() * 8 + plan.combine.size() * 16);
     put(k, static_cast<uint32_t>(step.kv_dtype));
     put(k, &step.common, sizeof(step.common));
     put(k, step.k_pool);
@@ -56,6 +56,7 @@ std::vector<uint8_t> plan_signature_bytes(const PagedAttentionStep& step, const 
         put(k, p.tile_first);
         put(k, p.tile_count);
         put(k, p.tiles_per_group);
+        put(k, p.part_heads);
         put(k, p.side);
         put(k, static_cast<uint32_t>(p.partial_offset));
         put(k, static_cast<uint32_t>(p.partial_offset >> 32));

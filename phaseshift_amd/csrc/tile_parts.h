@@ -1,0 +1,82 @@
+// Which tile launches run in two parts: a tile's even and odd 32-token chunks
+// on two waves per head, joined in LDS, and how many heads one workgroup
+// takes. Plain C++ (the launchers call it, the CPU tests hold it against
+// measured times of both kernels).
+#pragma once
+#include <cstdint>
+
+namespace psk {
+
+// A two-part launch's tiles of up to this many tokens run as one part: joining
+// the parts costs 1-2 us, about what splitting 8 chunks gains (FP8, 24/4 heads,
+// 6 per workgroup, 128 rows without context 15.1 us, in two parts 16.3; 512
+// rows 29.6 and 27.2).
+constexpr uint32_t kTwoPartTokens = 256;
+
+struct TileShape {
+    uint32_t head_dim;
+    uint32_t q_per_kv;
+    uint32_t kv_heads;
+    bool psq;
+    bool bf16;
+};
+
+// Heads per workgroup of an unsplit launch of implicit tiles (the prefill
+// launchers) of `rows` rows on `cus` CUs, 0 for one part.
+//
+// Such a launch has only tiles x kv_heads workgroups (units) and no scratch to
+// split K over, and its waves are bound by instruction issue: 5-6 one-head
+// waves load two of the four SIMDs twice, and up to 256 workgroups leave the
+// rest of the chip idle. In two parts 6 heads put 3 waves on every SIMD; where
+// the tiles alone do not reach the CUs the heads go to workgroups of 4 or 2.
+// Launcher times, one part -> two (us, 24/4 heads of 256; rows + context):
+//   FP8   48+0 12.5 -> 9.4 (2 heads)      BF16  128+1024 55.6 -> 42.8 (2)
+//   FP8   512+4096 166 -> 111 (4; 6: 122) PSQ4  512+4096 218 -> 172 (4; 6: 192)
+//   FP8   700+1024 69.3 -> 55.7 (6; 4: 81) PSQ8 1024+2048 157 -> 129 (6; 4: 207)
+//   FP8   2048+2048 262 -> 199 (6)        BF16  2048+0 154 -> 127 (6)
+// so the smallest workgroups that stay within one per CU win, then all heads.
+// A PSQ workgroup dequantizes for all its heads, so 2 of them pay only on a
+// nearly empty chip (8/1 heads of 128, PSQ8 128+1024: 4 heads 33.1, 2 34.9;
+// 48+0: 8.9 and 8.3).
+// Beyond one workgroup per CU: 5-6 heads always (SIMD
+// balance), 1-2 heads (the other waves have no head), 3-4 and 7-8 only where
+// one CU holds one one-part workgroup anyway (BF16 at 256, 16/4 heads 2048+2048
+// 289 -> 247; PSQ8 16/2 heads of 128, 4096+0 246 -> 185); FP8 and PSQ at 256
+// would lose (16/4 heads 2048+2048: FP8 156 -> 171, PSQ4 249 -> 266). 16 waves
+// (7-8 heads) need 128 registers a wave: head_dim <= 128.
+constexpr uint32_t implicit_part_heads(const TileShape& s, uint64_t rows, uint64_t cus) {
+    const uint32_t q = s.q_per_kv;
+    const bool wide = s.head_dim == 256u;
+    const uint64_t units = (rows + 15u) / 16u * s.kv_heads;
+    if (q <= 2u || units * ((q + 1u) / 2u) <= (s.psq ? cus / 4u : cus)) return 2u;
+    if (units * ((q + 3u) / 4u) <= cus) return 4u;
+    if (q == 5u || q == 6u) return 6u;
+    if (units > cus && !(wide ? s.bf16 : s.psq && q > 4u)) return 0u;
+    return q <= 4u ? 4u : wide ? 0u : 8u;
+}
+
+// The same for explicit tiles (verify blocks) and split launches: 6 for 5-6
+// heads, 0 otherwise. range: most tokens a workgroup reads (a split's, or the
+// longest visible range); units: workgroups with work.
+//
+// Whole verify calls (us, 24/4 heads of 256, one part -> two): FP8 8 blocks of
+// 16 rows over 2-16k tokens 56.3 -> 52.5, 32 over 2-8k 165 -> 157; unsplit, 16
+// of 12 rows over 256-2000 tokens 79.2 -> 63.1; BF16 61.7 -> 59.4, 221 -> 214. Over short ranges the second half
+// of the waves only costs its start: 8 blocks over 252 tokens 20.5 -> 22.3, 256
+// over 76 63.1 -> 71.6, and ranges up to 320 gain nothing (BF16 1.00-1.02x).
+// Heads below 256 leave room for several one-part workgroups on a CU: two parts
+// lose beyond one workgroup per CU (24/4 heads of 128, 128 blocks over 516
+// tokens, FP8 37.5 -> 44.5; at 32 past two per CU) and on splits up to 512 tokens
+// (16 blocks over 0.3-4k, 368 a split: 1.06-1.12x). PSQ gains from splits past
+// 512 tokens (PSQ4 32 blocks 211 -> 199; 272 tokens lose 3 us of 32-41);
+// unsplit its 8 one-part waves share the dequantization.
+constexpr uint32_t explicit_part_heads(const TileShape& s, bool split, uint64_t range, uint64_t units,
+                                       uint64_t cus) {
+    if (s.q_per_kv != 5u && s.q_per_kv != 6u) return 0u;
+    if (s.psq && !split) return 0u;
+    const bool wide = s.head_dim == 256u;
+    if (range <= (s.psq || (split && !wide) ? 2u * kTwoPartTokens : kTwoPartTokens + 64u)) return 0u;
+    return wide || units <= (s.head_dim == 32u ? 2u * cus : cus) ? 6u : 0u;
+}
+
+}  // namespace psk

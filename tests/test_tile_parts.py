@@ -1,0 +1,70 @@
+"""The rules that run tile launches in one part or in two
+(phaseshift_amd/csrc/tile_parts.h) against both kernels' times over the shapes
+they decide on (tests/measured/tile_parts_times_mi355x.json), and what the step
+planner makes of them. No GPU."""
+import json
+import os
+import subprocess
+
+import pytest
+
+from phaseshift_amd import KV_BF16, KV_FP8, state
+from tests.test_planner import args
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+# two runs of one build differ by up to 2-3% on calls of 10-30 us
+NOISE = 1.03
+
+
+def measured(kind):
+    with open(os.path.join(HERE, "measured", "tile_parts_times_mi355x.json")) as f:
+        return json.load(f)[kind]["times"]
+
+
+@pytest.fixture(scope="module")
+def rule(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("native") / "tile_parts_rule"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "phaseshift_amd", "csrc"),
+                    os.path.join(HERE, "native", "tile_parts_rule.cpp"), "-o", str(exe)], check=True)
+
+    def ask(lines):
+        r = subprocess.run([str(exe)], input="\n".join(lines), capture_output=True, text=True, check=True)
+        return [int(x) for x in r.stdout.split()]
+    return ask
+
+
+def flags(kv):
+    return f"{int(kv.startswith('psq'))} {int(kv == 'bf16')}"
+
+
+def test_explicit_rule_against_measured_times(rule):
+    rows = measured("explicit")
+    heads = rule(f"e {flags(kv)} {D} {q} {kvh} {split} {rng} {units}" for kv, D, q, kvh, split, rng, units, _, _ in rows)
+    assert len(heads) == len(rows)
+    for h, r in zip(heads, rows):
+        one, two = r[-2:]
+        assert not h or two <= NOISE * one, (h, r)
+        # 24/4 heads of 256 keep what two parts gain
+        if r[1] == 256 and not r[0].startswith("psq") and two < 0.95 * one:
+            assert h == 6, r
+
+
+def test_explicit_rule_takes_five_and_six_heads_only(rule):
+    heads = rule(f"e 0 0 256 {q} 4 0 2000 64" for q in range(1, 9))
+    assert heads == [0, 0, 0, 0, 6, 6, 0, 0]
+
+
+@pytest.mark.parametrize("kv", [KV_BF16, KV_FP8])
+def test_plan_signature_follows_the_parts(kv):
+    """A captured step runs the kernel its capture chose: the signature changes
+    where the choice does (a short verify range that grows past the line), and
+    only there."""
+    a = args(128)
+
+    def sig(visible):
+        reqs = [(16 * i, 16, 1, visible) for i in range(8)]
+        return state.plan_signature(a, kv, reqs, visible, 0, 0, 16, 16, 16, 16)
+    assert sig(100) == sig(252) == sig(320)
+    assert sig(321) == sig(1500)
+    assert sig(320) != sig(321)
