@@ -38,21 +38,41 @@ struct TileShape {
 // A PSQ workgroup dequantizes for all its heads, so 2 of them pay only on a
 // nearly empty chip (8/1 heads of 128, PSQ8 128+1024: 4 heads 33.1, 2 34.9;
 // 48+0: 8.9 and 8.3).
-// Beyond one workgroup per CU: 5-6 heads always (SIMD
-// balance), 1-2 heads (the other waves have no head), 3-4 and 7-8 only where
-// one CU holds one one-part workgroup anyway (BF16 at 256, 16/4 heads 2048+2048
-// 289 -> 247; PSQ8 16/2 heads of 128, 4096+0 246 -> 185); FP8 and PSQ at 256
-// would lose (16/4 heads 2048+2048: FP8 156 -> 171, PSQ4 249 -> 266). 16 waves
-// (7-8 heads) need 128 registers a wave: head_dim <= 128.
+//
+// Where two parts lose (times one part -> two as above; the lines lie where
+// the sign changes in the recorded times that the tests hold):
+// - Few heads over a short range: the launch does not know its context, but more
+//   than kTwoPartTokens rows always reach past it. Up to 2 heads 128+0 1.03-1.08x
+//   slower, 17+0 up to 1.19x (PSQ4, 8/4 heads of 256), the same for 3 (PSQ) and
+//   up to 4 (heads of 32 and 64); PSQ with 4 heads loses on 17 rows only, and with
+//   5, dequantized by workgroups of 4 and 1, on 128+0 (PSQ4 1.05x).
+// - Beyond one workgroup per CU. PSQ with 1-2 heads dequantizes for half the
+//   waves (8/8 heads of 256, 4000+0: PSQ4 522 -> 696; of 128, where a CU holds
+//   two, past 2 per CU 249 -> 295). 3-4 heads gain only in BF16 at 256 (16/4
+//   heads 2060+2048 392 -> 340; FP8 2048+2048 156 -> 171). 5-6 heads gain at 256 in every
+//   format, at 128 in BF16 and FP8 (24/4 heads 4000+0 0.84-0.86x; 5 heads lose
+//   2-4% between one and three workgroups per CU), in FP8 at 64 up to two per CU
+//   (20/4 heads 2040+0 0.97x, 2060+2048 1.07x) and in BF16 at 32; PSQ at 128
+//   (24/8 heads 1024+1024 1.03-1.06x, 4000+0 1.13-1.16x) and BF16 at 64 (24/8
+//   heads 1.02-1.11x) lose. 7-8 heads lose (32/4 heads of 128, PSQ 1.04-1.13x).
+// 16 waves (7-8 heads) need 128 registers a wave: head_dim <= 128.
 constexpr uint32_t implicit_part_heads(const TileShape& s, uint64_t rows, uint64_t cus) {
-    const uint32_t q = s.q_per_kv;
-    const bool wide = s.head_dim == 256u;
+    const uint32_t q = s.q_per_kv, D = s.head_dim;
     const uint64_t units = (rows + 15u) / 16u * s.kv_heads;
-    if (q <= 2u || units * ((q + 1u) / 2u) <= (s.psq ? cus / 4u : cus)) return 2u;
+    const bool few = q <= 2u || (s.psq ? q == 3u : q <= 4u && D <= 64u);
+    if (rows <= (few ? kTwoPartTokens : s.psq && q == 4u ? 32u : 0u)) return 0u;
+    if (q <= 2u) return !s.psq || units <= (D == 256u ? cus : 2u * cus) ? 2u : 0u;
+    if (units * ((q + 1u) / 2u) <= (s.psq ? cus / 4u : cus)) return 2u;
+    if (s.psq && q == 5u && rows <= kTwoPartTokens) return 0u;
     if (units * ((q + 3u) / 4u) <= cus) return 4u;
-    if (q == 5u || q == 6u) return 6u;
-    if (units > cus && !(wide ? s.bf16 : s.psq && q > 4u)) return 0u;
-    return q <= 4u ? 4u : wide ? 0u : 8u;
+    if (q == 5u || q == 6u) {
+        const bool gains = D == 256u || units <= cus ||
+                           (!s.psq && (D == 128u ? q == 6u || units > 3u * cus
+                                                 : s.bf16 ? D == 32u : units <= 2u * cus));
+        return gains ? 6u : 0u;
+    }
+    if (q <= 4u) return units <= cus || (D == 256u && s.bf16) ? 4u : 0u;
+    return units <= cus && D < 256u ? 8u : 0u;
 }
 
 // The same for explicit tiles (verify blocks) and split launches: 6 for 5-6

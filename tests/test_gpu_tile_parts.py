@@ -25,7 +25,8 @@ pytestmark = pytest.mark.gpu
     (24, 4, 256, 24, 700, 500),   # 4 heads, straddling pages
     (20, 4, 256, 16, 90, 520),    # 5 heads on 6
     (16, 2, 128, 16, 40, 1040),   # 8 heads
-    (4, 4, 128, 16, 280, 33),     # 1 head on 2
+    (4, 4, 128, 16, 280, 33),     # 1 head, few rows: one part
+    (4, 4, 128, 16, 280, 300),    # 1 head on 2
     (32, 4, 256, 16, 300, 100),   # 8 heads at 256: workgroups of 2 or 4
 ])
 def test_two_part_tiles(dev, kv, qh, kvh, D, page, prefix, rows):

@@ -68,3 +68,15 @@ def test_plan_signature_follows_the_parts(kv):
     assert sig(100) == sig(252) == sig(320)
     assert sig(321) == sig(1500)
     assert sig(320) != sig(321)
+
+
+def test_implicit_rule_against_measured_times(rule):
+    rows = measured("implicit")
+    heads = rule(f"i {flags(kv)} {D} {q} {kvh} {n}" for kv, D, q, kvh, n, _, _, _ in rows)
+    assert len(heads) == len(rows)
+    slower = [(h, r) for h, r in zip(heads, rows) if h and r[-1] > NOISE * r[-2]]
+    assert not slower, slower
+    for h, r in zip(heads, rows):
+        # the serving geometries keep what two parts gain
+        if (r[2], r[1]) in ((6, 256), (4, 256), (8, 128)) and r[-1] < 0.94 * r[-2]:
+            assert h or r[4] <= 32, r
