@@ -912,18 +912,26 @@ __global__ __launch_bounds__(NW * 64, waves_per_simd<FMT>()) void paged_decode_k
 // Combine of the split partials: workgroup = (row, kv_head, query head of the
 // group), O = sum_s W_s A_s / sum_s W_s l_s with W_s = e^(m_s - max m). The
 // launch is a chain of memory latencies, not bandwidth, so it is kept short:
-// every wave loads the (m, l) of all splits (lane = split) and derives the
-// weights itself, without a barrier; the splits go round the waves (and the lane
-// groups of a head_dim below 256), 16 B per lane, four loads in flight issued
-// before the weights are known; one barrier joins the waves' sums. Against a
-// thread per dim after two barriers, whole calls: one FP8 row of 4k tokens (24/4
-// heads of 256) 16.3 -> 14.8 us, 16 rows 32.1 -> 29.9, 24 PSQ4 rows 55.8 -> 53.9;
-// 8 waves equal it there and lose on many rows (8 verify blocks of 16 rows 58 us
-// against 55.5), 16 lose everywhere.
+// every wave loads the (m, l) of the splits (lane = split) and derives the
+// weights itself, without a barrier; the splits go round lane groups of
+// LANES = head_dim / 4 lanes, 16 B per lane, U loads in flight issued before the
+// weights are known; one barrier joins the groups' sums. With LANES known the
+// group indexes and the join are constants; up to 16 lanes one wave covers
+// several splits and a wave without any leaves at once. Launches of their own
+// (us; a thread per dim after two barriers | one kernel for every head_dim | this;
+// 24/4 heads): head_dim 256, 1 row of 16 splits 4.06 | 3.62 | 3.58, 128 rows 14.5 |
+// 12.8 | 12.8, 1 row of 200 splits 9.7 | 13.5 | 8.7; 512 rows of 9 splits at head_dim
+// 256 30.6 | 25.4 | 25.6, at 32 21.8 | 22.9 | 15.9. 8 waves a workgroup lose on many
+// rows, 16 everywhere.
 typedef f32x4 f32x4_a4 __attribute__((aligned(4)));   // the layout aligns rows to 8 B only
 
+template <int LANES>
 __global__ __launch_bounds__(kThreads) void split_reduce_kernel(const DecodeParams p) {
-    constexpr int U = 4;   // splits in flight per lane group
+    constexpr uint32_t lanes = LANES, step = kThreads / LANES;   // step: lane groups
+    // splits in flight per lane group; U * step divides 64, so a pass stays in
+    // one block of 64 splits
+    constexpr int U = step <= 16u ? 4 : 64 / (int)step;
+    constexpr bool kIdle = LANES <= 16;
     __shared__ f32x4 sums[kThreads];
     const psk_paged_attention_args& a = p.a;
     const uint32_t qpk = a.q_heads / a.kv_heads;
@@ -936,12 +944,15 @@ __global__ __launch_bounds__(kThreads) void split_reduce_kernel(const DecodePara
     if (n_used == 0u) return;   // the clamps below need one split
     const uint32_t stride = qpk * (2u + kPagedAttentionHeadLimit);
     const float* base = p.partials + (uint64_t)(row * a.kv_heads + kv_head) * p.splits * stride;
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t D = a.head_dim;
+    if constexpr (kIdle) {
+        // neither splits nor outputs (the barrier below does not wait for it)
+        const uint32_t first = __builtin_amdgcn_readfirstlane(tid & ~63u);
+        if (first >= D && first >= n_used * lanes) return;
+    }
 
-    // lane group of `lanes` lanes = one split's D values (4 per lane)
-    const uint32_t lanes = D <= 32u ? 8u : D <= 64u ? 16u : D <= 128u ? 32u : 64u;
-    const uint32_t s0 = tid / lanes, step = kThreads / lanes;
+    const uint32_t s0 = tid / lanes;
     const float* A = base + 2u * qpk + h * kPagedAttentionHeadLimit + 4u * (lane & (lanes - 1u));
     auto load = [&](uint32_t s) __attribute__((always_inline)) {
         return (f32x4)*reinterpret_cast<const f32x4_a4*>(A + (uint64_t)min(s, n_used - 1u) * stride);
@@ -962,8 +973,8 @@ __global__ __launch_bounds__(kThreads) void split_reduce_kernel(const DecodePara
     }
     gm = wave_max(gm);
     if (__any(bad)) return;   // the same in every wave
-    const float w0 = __expf(m0 - gm);
-    float L = lane < n_used ? w0 * l0 : 0.0f;
+    float w = __expf(m0 - gm);   // of the current block of 64 splits, lane = split
+    float L = lane < n_used ? w * l0 : 0.0f;
     for (uint32_t s = lane + 64u; s < n_used; s += 64u)
         L += __expf(base[(uint64_t)s * stride + h] - gm) * base[(uint64_t)s * stride + qpk + h];
     L = wave_sum(L);
@@ -977,12 +988,12 @@ __global__ __launch_bounds__(kThreads) void split_reduce_kernel(const DecodePara
 #pragma unroll
             for (int u = 0; u < U; ++u) x[u] = load(sb + s0 + (U + u) * step);
         }
+        if (sb != 0u && (sb & 63u) == 0u) w = __expf(base[(uint64_t)min(sb + lane, n_used - 1u) * stride + h] - gm);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t s = sb + s0 + u * step;
-            float w = __shfl(w0, (int)(s & 63u), 64);
-            if (s >= 64u && s < n_used) w = __expf(base[(uint64_t)s * stride + h] - gm);
-            if (s < n_used) O += w * y[u];
+            const float ws = __shfl(w, (int)(s & 63u), 64);
+            if (s < n_used) O += ws * y[u];
         }
     }
     sums[tid] = O;
@@ -990,7 +1001,13 @@ __global__ __launch_bounds__(kThreads) void split_reduce_kernel(const DecodePara
     if (tid >= D) return;
     const float* part = reinterpret_cast<const float*>(sums);
     float o = 0.0f;
-    for (uint32_t i = 0; i < step; ++i) o += part[i * 4u * lanes + tid];
+    if constexpr (kIdle) {
+        const uint32_t groups = min(step, n_used);   // the others hold no split
+        for (uint32_t i = 0; i < groups; ++i) o += part[i * 4u * lanes + tid];
+    } else {
+#pragma unroll
+        for (uint32_t i = 0; i < step; ++i) o += part[i * 4u * lanes + tid];
+    }
     const uint64_t oi = (uint64_t)row * a.output_row_stride + (uint64_t)(kv_head * qpk + h) * D + tid;
     const float res = o / L;
     if (a.output_dtype == PSK_OUT_F32)
@@ -1106,7 +1123,12 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream) {
 hipError_t launch_reduce(const DecodeParams& p, hipStream_t stream) {
     const uint64_t grid = (uint64_t)p.a.rows * p.a.q_heads;
     if (grid == 0u || grid > 0x7FFFFFFFull) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(split_reduce_kernel, dim3((uint32_t)grid), dim3(kThreads), 0, stream, p);
+    const uint32_t D = p.a.head_dim;
+    auto* const kernel = D <= 32u    ? split_reduce_kernel<8>
+                         : D <= 64u  ? split_reduce_kernel<16>
+                         : D <= 128u ? split_reduce_kernel<32>
+                                     : split_reduce_kernel<64>;
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)grid), dim3(kThreads), 0, stream, p);
     return hipGetLastError();
 }
 

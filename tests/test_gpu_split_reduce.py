@@ -133,3 +133,16 @@ def test_split_reduce_leaves_rows_without_splits_unwritten(dev):
     want = oracle.split_reduce(geom, part[keep], splits, used[keep], np.zeros(len(keep), np.uint32), len(keep))
     np.testing.assert_allclose(got[keep], want, rtol=2e-5, atol=2e-5 * np.abs(want).max())
     assert np.all(got[used == 0] == 7.0)
+
+
+@pytest.mark.parametrize("D", [8, 32, 40, 64, 128, 256])
+@pytest.mark.parametrize("splits", [1, 3, 9, 33, 64, 65, 130, 260])
+def test_split_reduce_lane_groups(dev, splits, D):
+    """Every lane-group width (8 lanes up to head_dim 32, 16, 32, 64), around the
+    splits where waves go idle (few splits) and where the weights move to the
+    next block of 64. Tolerance as above: the order of the fp32 sum is the only
+    difference, at most 260 terms of 2^-24 relative."""
+    c = reduce_case(5, splits, D, 10 * splits + D, pps=1)
+    got = run_reduce(dev, c, splits)
+    want = oracle_reduce(c, splits)
+    np.testing.assert_allclose(got, want, rtol=2e-5, atol=2e-5 * np.abs(want).max())
