@@ -9,6 +9,7 @@ import subprocess
 import pytest
 
 from phaseshift_amd import KV_BF16, KV_FP8, state
+from tests.test_gpu_tile_parts import SPLIT_CASES
 from tests.test_planner import args
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -53,6 +54,13 @@ def test_explicit_rule_against_measured_times(rule):
 def test_explicit_rule_takes_five_and_six_heads_only(rule):
     heads = rule(f"e 0 0 256 {q} 4 0 2000 64" for q in range(1, 9))
     assert heads == [0, 0, 0, 0, 6, 6, 0, 0]
+
+
+def test_split_tiles_of_the_gpu_test_take_two_parts(rule):
+    """The shapes that tests/test_gpu_tile_parts.py runs for two parts have them."""
+    lines = [f"e {flags(kv)} {D} {qh // kvh} {kvh} 1 {pps * page} {len(lens) * kvh * splits}"
+             for kvs, qh, kvh, D, page, lens, splits, pps in SPLIT_CASES for kv in kvs]
+    assert rule(lines) == [6] * len(lines)
 
 
 @pytest.mark.parametrize("kv", [KV_BF16, KV_FP8])
