@@ -967,7 +967,10 @@ constexpr size_t tile_pg_lds_bytes() {
 // the HPW = 2 heads of the workgroup's head pair. RT == 1 (verify blocks,
 // implicit tiles, other group sizes): the NW waves own HPW = 1 head each of
 // one tile. The first 4 waves issue the DMAs; the first 4 (8 at head_dim
-// 256 with 8 waves) dequantize.
+// 256 with 8 waves) dequantize. TS == 2: a stage holds both chunks of a pair,
+// and the first 8 waves do both, four per chunk (4 waves: for two chunks each).
+// At head_dim 256 the two-part kernels spill 2-13 registers (4 and 8 waves:
+// PSQ8 2-10, PSQ4 8-13; 12 waves 9-10), the one-part ones 1-6.
 template <int FMT, int D, int NW, int HPW, int RT, int TS, bool kAl16>
 __global__ __launch_bounds__(NW * 64, tile_waves_per_simd(HPW, NW)) void paged_tile_psq_group_kernel(const TileParams p) {
     constexpr int WH = NW / RT / TS;                  // waves along the heads of one tile

@@ -79,11 +79,18 @@ constexpr uint32_t implicit_part_heads(const TileShape& s, uint64_t rows, uint64
 // heads, 0 otherwise. range: most tokens a workgroup reads (a split's, or the
 // longest visible range); units: workgroups with work.
 //
-// Whole verify calls (us, 24/4 heads of 256, one part -> two): FP8 8 blocks of
-// 16 rows over 2-16k tokens 56.3 -> 52.5, 32 over 2-8k 165 -> 157; unsplit, 16
-// of 12 rows over 256-2000 tokens 79.2 -> 63.1; BF16 61.7 -> 59.4, 221 -> 214. Over short ranges the second half
+// Whole verify calls repeated on the same buffers, whose K/V the last-level
+// cache then holds (us, 24/4 heads of 256, one part -> two): FP8 8 blocks of 16
+// rows over 2-16k tokens 56.3 -> 52.5, 32 over 2-8k 165 -> 157; unsplit, 16 of 12
+// rows over 256-2000 tokens 79.2 -> 63.1; BF16 61.7 -> 59.4, 221 -> 214. With K/V
+// read from HBM (600 MB of other reads before each call; call times with their
+// launch) the first gains 63.3 -> 61.4, 32 FP8 blocks over 1.6-6.8k 119.6 -> 110.2
+// (cached 116.6 -> 101.4), 17 BF16 blocks of 14 rows over 424-1594 86.8 -> 75.8,
+// and of 43 drawn verify calls none is slower by more than 1.3%, what calls of
+// the same kernel differ by. Over short ranges the second half
 // of the waves only costs its start: 8 blocks over 252 tokens 20.5 -> 22.3, 256
 // over 76 63.1 -> 71.6, and ranges up to 320 gain nothing (BF16 1.00-1.02x).
+// Other group sizes stay one part: they were not measured in two here.
 // Heads below 256 leave room for several one-part workgroups on a CU: two parts
 // lose beyond one workgroup per CU (24/4 heads of 128, 128 blocks over 516
 // tokens, FP8 37.5 -> 44.5; at 32 past two per CU) and on splits up to 512 tokens
