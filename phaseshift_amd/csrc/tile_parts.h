@@ -44,8 +44,11 @@ struct TileShape {
 // - Few heads over a short range: the launch does not know its context, but more
 //   than kTwoPartTokens rows always reach past it. Up to 2 heads 128+0 1.03-1.08x
 //   slower, 17+0 up to 1.19x (PSQ4, 8/4 heads of 256), the same for 3 (PSQ) and
-//   up to 4 (heads of 32 and 64); PSQ with 4 heads loses on 17 rows only, and with
+//   up to 4 (heads of 32 and 64); PSQ with 4 heads loses on 17 rows, and with
 //   5, dequantized by workgroups of 4 and 1, on 128+0 (PSQ4 1.05x).
+// - The 16-wave workgroups of 7-8 heads start slower: 64/8 heads of 128, 260+0
+//   FP8 16.6 -> 18.5, BF16 16.3 -> 17.8, PSQ8 290+0 21.3 -> 22.6; level from 400 rows
+//   (PSQ, BF16) and 520 (FP8); of 64, FP8 800+0 24.2 -> 25.1, level at 1000.
 // - Beyond one workgroup per CU. PSQ with 1-2 heads dequantizes for half the
 //   waves (8/8 heads of 256, 4000+0: PSQ4 522 -> 696; of 128, where a CU holds
 //   two, past 2 per CU 249 -> 295). 3-4 heads gain only in BF16 at 256 (16/4
@@ -72,7 +75,7 @@ constexpr uint32_t implicit_part_heads(const TileShape& s, uint64_t rows, uint64
         return gains ? 6u : 0u;
     }
     if (q <= 4u) return units <= cus || (D == 256u && s.bf16) ? 4u : 0u;
-    return units <= cus && D < 256u ? 8u : 0u;
+    return units <= cus && D < 256u && rows > (D <= 64u ? 896u : s.psq || s.bf16 ? 384u : 512u) ? 8u : 0u;
 }
 
 // The same for explicit tiles (verify blocks) and split launches: 6 for 5-6

@@ -86,5 +86,5 @@ def test_implicit_rule_against_measured_times(rule):
     assert not slower, slower
     for h, r in zip(heads, rows):
         # the serving geometries keep what two parts gain
-        if (r[2], r[1]) in ((6, 256), (4, 256), (8, 128)) and r[-1] < 0.94 * r[-2]:
+        if (r[2], r[1]) in ((6, 256), (4, 256), (8, 128)) and r[3] <= 4 and r[-1] < 0.94 * r[-2]:
             assert h or r[4] <= 32, r
