@@ -45,7 +45,11 @@ struct TileShape {
 //   than kTwoPartTokens rows always reach past it. Up to 2 heads 128+0 1.03-1.08x
 //   slower, 17+0 up to 1.19x (PSQ4, 8/4 heads of 256), the same for 3 (PSQ) and
 //   up to 4 (heads of 32 and 64); PSQ with 4 heads loses on 17 rows, and with
-//   5, dequantized by workgroups of 4 and 1, on 128+0 (PSQ4 1.05x).
+//   5, dequantized by workgroups of 4 and 1, on 128+0 (PSQ4 1.05x). PSQ with 4 heads
+//   of 256 on 33-256 rows takes pairs, also past a quarter of the CUs (PSQ4 16/4
+//   heads: 140+0 17.7 -> 18.6, in fours 19.8; 140+333 32.9 -> 29.6, 31.4;
+//   140+2900 150 -> 118, 119): it loses up to 7% without context and gains
+//   6-25% from 256 tokens of it, so two parts stay.
 // - The 16-wave workgroups of 7-8 heads start slower: 64/8 heads of 128, 260+0
 //   FP8 16.6 -> 18.5, BF16 16.3 -> 17.8, PSQ8 290+0 21.3 -> 22.6; level from 400 rows
 //   (PSQ, BF16) and 520 (FP8); of 64, FP8 800+0 24.2 -> 25.1, level at 1000.
@@ -65,7 +69,8 @@ constexpr uint32_t implicit_part_heads(const TileShape& s, uint64_t rows, uint64
     const bool few = q <= 2u || (s.psq ? q == 3u : q <= 4u && D <= 64u);
     if (rows <= (few ? kTwoPartTokens : s.psq && q == 4u ? 32u : 0u)) return 0u;
     if (q <= 2u) return !s.psq || units <= (D == 256u ? cus : 2u * cus) ? 2u : 0u;
-    if (units * ((q + 1u) / 2u) <= (s.psq ? cus / 4u : cus)) return 2u;
+    const bool pairs = !s.psq || (q == 4u && D == 256u && rows <= kTwoPartTokens);
+    if (units * ((q + 1u) / 2u) <= (pairs ? cus : cus / 4u)) return 2u;
     if (s.psq && q == 5u && rows <= kTwoPartTokens) return 0u;
     if (units * ((q + 3u) / 4u) <= cus) return 4u;
     if (q == 5u || q == 6u) {

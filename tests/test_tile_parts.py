@@ -82,8 +82,16 @@ def test_implicit_rule_against_measured_times(rule):
     rows = measured("implicit")
     heads = rule(f"i {flags(kv)} {D} {q} {kvh} {n}" for kv, D, q, kvh, n, _, _, _ in rows)
     assert len(heads) == len(rows)
-    slower = [(h, r) for h, r in zip(heads, rows) if h and r[-1] > NOISE * r[-2]]
+    # PSQ with 4 heads on few rows: a launch that may or may not have a context
+    # (it does not know) gains 6-25% with 256 tokens of it or more, for up to 7% without
+    mixed = [r for r in rows if r[0].startswith("psq") and r[2] == 4 and r[4] <= 256]
+    slower = [(h, r) for h, r in zip(heads, rows)
+              if h and r[-1] > (1.075 if r in mixed and r[5] < 256 else NOISE) * r[-2]]
     assert not slower, slower
+    assert rule(["i 1 0 256 4 4 140", "i 1 0 256 4 8 256", "i 1 0 256 4 4 257"]) == [2, 2, 4]
+    for r in mixed:
+        if r[1] == 256 and r[4] > 32 and r[5] >= 256:
+            assert r[-1] < 0.95 * r[-2], r
     for h, r in zip(heads, rows):
         # the serving geometries keep what two parts gain
         if (r[2], r[1]) in ((6, 256), (4, 256), (8, 128)) and r[3] <= 4 and r[-1] < 0.94 * r[-2]:
