@@ -53,6 +53,10 @@ struct TileShape {
 // - The 16-wave workgroups of 7-8 heads start slower: 64/8 heads of 128, 260+0
 //   FP8 16.6 -> 18.5, BF16 16.3 -> 17.8, PSQ8 290+0 21.3 -> 22.6; level from 400 rows
 //   (PSQ, BF16) and 520 (FP8); of 64, FP8 800+0 24.2 -> 25.1, level at 1000.
+// - BF16 heads of 128 in groups of 1-2, just below three workgroups per CU (16/8
+//   heads, 1500 rows: +0 60.5 -> 57.9, +1000 109 -> 113, +2900 199 -> 214; at 2.65
+//   and 3.05 per CU two parts gain 2-9%, and so they do at 2.97 on 4 KV heads, whose
+//   3036 rows differ more in length).
 // - Beyond one workgroup per CU. PSQ with 1-2 heads dequantizes for half the
 //   waves (8/8 heads of 256, 4000+0: PSQ4 522 -> 696; of 128, where a CU holds
 //   two, past 2 per CU 249 -> 295). 3-4 heads gain only in BF16 at 256 (16/4
@@ -68,6 +72,8 @@ constexpr uint32_t implicit_part_heads(const TileShape& s, uint64_t rows, uint64
     const uint64_t units = (rows + 15u) / 16u * s.kv_heads;
     const bool few = q <= 2u || (s.psq ? q == 3u : q <= 4u && D <= 64u);
     if (rows <= (few ? kTwoPartTokens : s.psq && q == 4u ? 32u : 0u)) return 0u;
+    if (q <= 2u && s.bf16 && D == 128u && rows < 2048u && 10u * units > 27u * cus && units <= 3u * cus)
+        return 0u;
     if (q <= 2u) return !s.psq || units <= (D == 256u ? cus : 2u * cus) ? 2u : 0u;
     const bool pairs = !s.psq || (q == 4u && D == 256u && rows <= kTwoPartTokens);
     if (units * ((q + 1u) / 2u) <= (pairs ? cus : cus / 4u)) return 2u;
